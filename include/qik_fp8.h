@@ -129,7 +129,7 @@ int qik_fp8_gemm_ws(const qik_fp8_gemm_args* args, void* workspace, int64_t work
  * tile rows, small tile columns, 1 when the small tiles' workgroups come
  * first in blockIdx order, the number of K slices (1: no split); *n1 = the
  * output columns [0, n1) the big tiles cover (N for a K split, which runs
- * 128 x 128 tiles only).  QIK_ERR_SHAPE for a shape qik_fp8_gemm_validate
+ * one tile shape).  QIK_ERR_SHAPE for a shape qik_fp8_gemm_validate
  * refuses (with its strides equal to K, K and N). */
 int qik_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, int32_t cus, int32_t* plan, int64_t* n1);
 

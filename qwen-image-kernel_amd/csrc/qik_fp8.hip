@@ -19,9 +19,9 @@
 // BM x BN tile of out^T = W . A^T (MFMA A operand = weight rows n, B operand
 // = activation rows m), so each lane ends with 4 consecutive n of one row m
 // per register quad.  Tiles of A and W reach LDS directly
-// (buffer_load_dwordx4 ... lds, no register staging), 64 or 128 k-bytes per
-// stage, ahead of their use, with a 16-byte chunk swizzle that makes the
-// fragment reads conflict-free; each wave reads the next fragments while its
+// (buffer_load_dwordx4 ... lds, no register staging), 128 k-bytes per stage,
+// two to four stages ahead of their use, with a 16-byte chunk swizzle that
+// makes the fragment reads conflict-free; each wave reads the next fragments while its
 // MFMAs run on the current ones, and the copies are issued between the MFMAs.
 // The outputs go out through LDS as whole rows.  Workgroups map to tiles XCD
 // by XCD (the dispatcher deals workgroup b to XCD b % 8), so one XCD's L2
@@ -483,8 +483,6 @@ __global__ void __launch_bounds__(QT) dequant_kernel(const unsigned char* w, con
 // GEMM
 // ---------------------------------------------------------------------------
 
-constexpr int KB = 64;   // k bytes per stage (one MFMA k-step)
-
 // A range of output columns computed with one tile shape.
 struct GemmRegion {
   const unsigned char* w;  // weight row of the region's first column
@@ -509,45 +507,42 @@ struct GemmParams {
   float* partial;   // split launches: [ksplit][M][N] fp32 sums of each slice
 };
 
-template <int BM_, int BN_, int NS_, int WGM_ = 2, int WGN_ = 2>
-struct Cfg {
-  static constexpr int KB = qik_fp8::KB;
-  static constexpr int BM = BM_, BN = BN_, NS = NS_;
-  static constexpr int WGM = WGM_, WGN = WGN_;     // waves along m and n
+// Tile shape BM x BN, NS stages of 128 k-bytes (two MFMA k-steps per barrier;
+// each copied row a whole 128-byte line), WGM x WGN waves.  A stage's copies go
+// out NS steps ahead of its first fragment reads.
+//
+// What bounds a tile of the smaller shapes is the latency of those copies: at
+// two stages a step cannot be shorter than one L2 or HBM round trip (about
+// 0.9 us under load; the 192 x 128 tile took that long per step for 0.4 us of
+// MFMA and of copy path), so everything that leaves LDS for a third stage has
+// one.  Each against the shape that ran before it, on one box: 1728 x 3072 x
+// 12288 (M x N x K) 70 us against 97 (192 x 128, 3 stages against 2), 1152 x
+// 3072 x 12288 52 / 62 (128 x 128 against 6 stages of 64 k-bytes, whose rows
+// are half lines fetched twice), 768 x 9216 x 3072 25.0 / 26.8 and 1728 x 4096
+// x 4096 31.2 / 33.3 (256 x 128).  Three stages were 1-4% ahead of four and
+// five at 128 x 128 and 192 x 128 (a longer prologue for no shorter step); the
+// 64 x 64 tile (a step of two MFMAs) is 3-8% faster with four than with three.
+// 256 x 256 and 192 x 256 fill LDS with two stages, and their steps (1.5 and
+// 1.3 us) are longer than the round trip.
+template <int BM_, int BN_, int WGM_, int WGN_, int NS_>
+struct CfgK128 {
+  static constexpr int KB = 128, NS = NS_;
+  static constexpr int BM = BM_, BN = BN_;
+  static constexpr int WGM = WGM_, WGN = WGN_;        // waves along m and n
   static constexpr int NW = WGM * WGN, NT = 64 * NW;
   static constexpr int WM = BM / WGM, WN = BN / WGN;  // wave tile
   static constexpr int MI = WM / 32, NJ = WN / 32;
-  static constexpr int A_BYTES = BM * KB;          // A tile of one stage
-  static constexpr int STAGE = (BM + BN) * KB;
-  static constexpr int AI = BM / (16 * NW);        // 1 KiB copies of A per wave per stage
-  static constexpr int WI = BN / (16 * NW);
-  static constexpr int COPIES = AI + WI;
-  static_assert(NW == 4 || NW == 8, "one or two waves per SIMD");
-  static_assert(AI * 16 * NW == BM && WI * 16 * NW == BN, "whole copies per wave");
-  static_assert(MI * 32 == WM && NJ * 32 == WN, "whole MFMA blocks per wave");
-  static_assert(NS >= 3, "copies run at least two stages ahead");
-};
-
-// Tiles with 128 k-bytes per stage: two MFMA k-steps per barrier, and each
-// copied row a whole 128-byte line (at 64 bytes a row is half a line, fetched
-// by two stages).  Two stages: a stage's copies go out one step (two MFMA
-// k-steps) before its first fragment reads.
-template <int BM_, int BN_, int WGM_ = 2, int WGN_ = 4>
-struct CfgK128 {
-  static constexpr int KB = 128, NS = 2;
-  static constexpr int BM = BM_, BN = BN_;
-  static constexpr int WGM = WGM_, WGN = WGN_;
-  static constexpr int NW = WGM * WGN, NT = 64 * NW;
-  static constexpr int WM = BM / WGM, WN = BN / WGN;
-  static constexpr int MI = WM / 32, NJ = WN / 32;
-  static constexpr int A_BYTES = BM * KB;
+  static constexpr int A_BYTES = BM * KB;             // A tile of one stage
   static constexpr int STAGE = (BM + BN) * KB;
   static constexpr int AI = BM / (8 * NW);  // 1 KiB copies (8 rows) of A per wave per stage
   static constexpr int WI = BN / (8 * NW);
   static constexpr int COPIES = AI + WI;
   static_assert(NW == 4 || NW == 8, "one or two waves per SIMD");
+  static_assert(NS >= 2 && (NS - 1) * COPIES < 64, "the prologue's copies fit the vmcnt field");
+  static_assert(NS * STAGE <= 160 * 1024, "the stages fit LDS");
   static_assert(AI * 8 * NW == BM && WI * 8 * NW == BN, "whole copies per wave");
   static_assert(MI * 32 == WM && NJ * 32 == WN, "whole MFMA blocks per wave");
+  static_assert((BN & (BN - 1)) == 0, "the output staging's swizzle needs a power of two");
 };
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
@@ -578,13 +573,6 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (0x7 << 4) | (0x3f << 8));
 }
 
-// Layout of a stage in LDS: A rows [BM][64 B], then W rows [BN][64 B].  The
-// 16-byte chunk c of row r sits at physical chunk c ^ ((r >> 2) & 3): a
-// fragment read (32 rows, one chunk each per 32 lanes) then touches all 64
-// banks once per 16 lanes, and a 1 KiB copy (16 rows x 4 chunks) writes one
-// contiguous KiB.
-__device__ __forceinline__ int swz(int r) { return (r >> 2) & 3; }
-
 // Origin of the tile of workgroup bx of region rg (bx % 8 is the XCD: every
 // region starts at a multiple of 8): XCD x takes a contiguous run of the tile
 // order, which walks group_m tile rows at a time.  False for a padding
@@ -611,181 +599,29 @@ __device__ __forceinline__ void store_tile(const GemmParams& p, const GemmRegion
                                            const f32x16 (&acc)[C::NJ][C::MI], unsigned char* lds, const int wave,
                                            const int lane);
 
-// One BM x BN output tile of region g; bx counts the region's workgroups.
-// SPLIT: the workgroup sums k-steps [kb, ke) of slice `slice` and writes the
-// fp32 sums to p.partial instead of the outputs.
-template <class C, bool FP16, bool SPLIT = false>
-__device__ __forceinline__ void gemm_tile(const GemmParams& p, const GemmRegion& rg, const int bx,
-                                          unsigned char* lds, const int slice = 0) {
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: copy targets go to SGPRs
+// The fp32 sums of one k-slice of a tile into p.partial, 4 columns of one row
+// per lane and register quad.
+template <class C>
+__device__ __forceinline__ void store_partial(const GemmParams& p, const GemmRegion& rg, const int m0, const int n0,
+                                              const f32x16 (&acc)[C::NJ][C::MI], const int slice, const int wave,
+                                              const int lane) {
   const int wm = wave % C::WGM, wn = wave / C::WGM;
-
-  int m0, n0;
-  if (!tile_origin<C>(rg, bx, m0, n0)) return;
-  const int mrows = min(C::BM, p.M - m0);
-  const int nrows = min(C::BN, rg.N - n0);
-
-  // per-lane copy offsets: copy i of this wave fills 16-row group wave + NW i
-  // of its tile; lane l writes row l/4 of the group, physical chunk l%4,
-  // which holds logical chunk (l%4) ^ swz(row)
-  const int crow = wave * 16 + (lane >> 2);
-  const int cchunk = ((lane & 3) ^ ((lane >> 4) & 3)) * 16;
-  uint32_t aoff[C::AI], woff[C::WI];
+  float* dst = p.partial + (int64_t)slice * p.M * rg.N;
 #pragma unroll
-  for (int i = 0; i < C::AI; ++i) aoff[i] = (uint32_t)((crow + 16 * C::NW * i) * p.lda + cchunk);
+  for (int j = 0; j < C::NJ; ++j) {
 #pragma unroll
-  for (int i = 0; i < C::WI; ++i) woff[i] = (uint32_t)((crow + 16 * C::NW * i) * p.ldw + cchunk);
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)lds;
-  const unsigned char* abase = p.a + (int64_t)m0 * p.lda;
-  const unsigned char* wbase = rg.w + (int64_t)n0 * p.ldw;
-  const int nkall = (p.K + KB - 1) / KB;
-  const int kb = SPLIT ? (int)((int64_t)nkall * slice / p.ksplit) : 0;
-  const int nk = SPLIT ? (int)((int64_t)nkall * (slice + 1) / p.ksplit) : nkall;  // end of the k-steps
-
-  // copy state of one k-step: the stage's LDS address and the two buffer
-  // resources; past the end of K a lane's chunk would read the next row, so
-  // its offset gets the top bit (out of range: it lands as zeros)
-  struct StepCopies {
-    u32x4 ra, rw;
-    uint32_t st;
-    uint32_t dead;  // 0, or 0x80000000 for a lane whose chunk lies past K
-  };
-  // A k-step at or past the end (kt >= nk) gets empty resources: its copies
-  // fetch nothing and write zeros into a stage that no later step reads, so
-  // every step issues the same copies and the vmcnt waits stay uniform.
-  auto prepare = [&](const int kt) __attribute__((always_inline)) {
-    StepCopies sc;
-    const int koff = kt * KB;
-    const int lim = p.K - koff;  // k bytes left in every row
-    const int kin = min(KB, lim);
-    sc.ra = rsrc_words(abase + koff, kt < nk ? (uint32_t)((mrows - 1) * p.lda + kin) : 0u);
-    sc.rw = rsrc_words(wbase + koff, kt < nk ? (uint32_t)((nrows - 1) * p.ldw + kin) : 0u);
-    sc.st = lds0 + (uint32_t)((kt % C::NS) * C::STAGE);
-    sc.dead = (lim < KB && cchunk >= lim) ? 0x80000000u : 0u;
-    return sc;
-  };
-  // copy i of this wave's list (A copies first, then W)
-  auto issue = [&](const StepCopies& sc, const int i) __attribute__((always_inline)) {
-    if (i < C::AI) dma16(sc.ra, sc.st + (uint32_t)((wave + C::NW * i) * 1024), aoff[i] | sc.dead);
-    else dma16(sc.rw, sc.st + (uint32_t)(C::A_BYTES + (wave + C::NW * (i - C::AI)) * 1024), woff[i - C::AI] | sc.dead);
-  };
-  auto copy_stage = [&](const int kt) __attribute__((always_inline)) {
-    const StepCopies sc = prepare(kt);
+    for (int qd = 0; qd < 4; ++qd) {
+      const int n = n0 + wn * C::WN + j * 32 + qd * 8 + (lane >> 5) * 4;
 #pragma unroll
-    for (int i = 0; i < C::COPIES; ++i) issue(sc, i);
-  };
-
-  // fragment read offsets: lane l reads row l%32 of a 32-row block, logical
-  // chunks 2*(l/32) and 2*(l/32)+1
-  const int frow = lane & 31;
-  const uint32_t f0 = (uint32_t)(frow * KB + (((lane >> 5) * 2) ^ swz(frow)) * 16);
-  const uint32_t f1 = (uint32_t)(frow * KB + (((lane >> 5) * 2 + 1) ^ swz(frow)) * 16);
-  // half r % 2 of fragment r / 2 (A fragments first, then W) of stage kt
-  constexpr int NRD = 2 * (C::MI + C::NJ);
-  auto read_frag = [&](const int kt, const int r, i32x8 (&fa)[C::MI], i32x8 (&fw)[C::NJ])
-      __attribute__((always_inline)) {
-    const unsigned char* st = lds + (kt % C::NS) * C::STAGE;
-    const int f = r >> 1;
-    const uint32_t off = (r & 1) ? f1 : f0;
-    const unsigned char* b = f < C::MI ? st + (wm * C::WM + f * 32) * KB
-                                       : st + C::A_BYTES + (wn * C::WN + (f - C::MI) * 32) * KB;
-    const u32x4 v = *reinterpret_cast<const u32x4*>(b + off);
-    i32x8& dst = f < C::MI ? fa[f] : fw[f - C::MI];
-    const int e = (r & 1) * 4;
-    dst[e] = (int)v.x;
-    dst[e + 1] = (int)v.y;
-    dst[e + 2] = (int)v.z;
-    dst[e + 3] = (int)v.w;
-  };
-  auto read_frags = [&](const int kt, i32x8 (&fa)[C::MI], i32x8 (&fw)[C::NJ]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int r = 0; r < NRD; ++r) read_frag(kt, r, fa, fw);
-  };
-
-  f32x16 acc[C::NJ][C::MI];
-#pragma unroll
-  for (int j = 0; j < C::NJ; ++j)
-#pragma unroll
-    for (int i = 0; i < C::MI; ++i) acc[j][i] = f32x16{};
-
-  // prologue: stages 0 .. NS-2 in flight, stage 0 published, its fragments read
-#pragma unroll
-  for (int s0 = 0; s0 < C::NS - 1; ++s0) copy_stage(kb + s0);
-  wait_vmcnt<(C::NS - 2) * C::COPIES>();
-  __syncthreads();
-  i32x8 fa[2][C::MI], fw[2][C::NJ];
-  read_frags(kb, fa[0], fw[0]);
-
-  // k-step kt: publish stage kt+1 (its copies done, and every wave past its
-  // MFMAs of kt-1, so stage kt-1 = kt+NS-1 is free), then run the MFMAs of kt
-  // with the fragment reads of kt+1 between the first half of them and the
-  // copies of kt+NS-1 between the second half.  Issued as one burst, the 16
-  // reads of a 256 x 256 tile held the wave at its second MFMA while the
-  // matrix core idled.  sched_barrier(0) pins the order: the compiler would
-  // otherwise hoist the wait and barrier of the next step above this step's
-  // MFMAs and bunch the reads and copies together.  The reads of the step
-  // after the last (a stage whose contents are not used) are issued too, so
-  // the step stays one basic block.
-  auto step = [&](const int kt, const int cur) __attribute__((always_inline)) {
-    constexpr int NMF = C::NJ * C::MI;
-    // reads after MFMAs [0, H), copies after MFMAs [CB, NMF); a wave with a
-    // single MFMA per step (64 x 64 tiles) issues both after it
-    constexpr int H = NMF >= 2 ? NMF / 2 : 1;
-    constexpr int CB = NMF >= 2 ? H : 0;
-    constexpr int CN = NMF - CB;
-    __builtin_amdgcn_sched_barrier(0);
-    wait_vmcnt<(C::NS - 3) * C::COPIES>();
-    __syncthreads();
-    __builtin_amdgcn_sched_barrier(0);
-    const StepCopies sc = prepare(kt + C::NS - 1);
-#pragma unroll
-    for (int idx = 0; idx < NMF; ++idx) {
-      const int j = idx / C::MI, i = idx % C::MI;
-      acc[j][i] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fw[cur][j], fa[cur][i], acc[j][i], 0, 0, 0, 0,
-                                                                   0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      if (idx < H) {
-#pragma unroll
-        for (int r = idx * NRD / H; r < (idx + 1) * NRD / H; ++r) read_frag(kt + 1, r, fa[cur ^ 1], fw[cur ^ 1]);
-      }
-      if (idx >= CB) {
-#pragma unroll
-        for (int c = (idx - CB) * C::COPIES / CN; c < (idx - CB + 1) * C::COPIES / CN; ++c) issue(sc, c);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
-  int kt = kb;
-  for (; kt + 1 < nk; kt += 2) {
-    step(kt, 0);
-    step(kt + 1, 1);
-  }
-  if (kt < nk) step(kt, 0);
-
-  wait_vmcnt<0>();  // the copies of the steps past the end still land in their stages
-  if constexpr (SPLIT) {
-    // the slice's fp32 sums, 4 columns of one row per lane and register quad
-    float* dst = p.partial + (int64_t)slice * p.M * rg.N;
-#pragma unroll
-    for (int j = 0; j < C::NJ; ++j) {
-#pragma unroll
-      for (int qd = 0; qd < 4; ++qd) {
-        const int n = n0 + wn * C::WN + j * 32 + qd * 8 + (lane >> 5) * 4;
-#pragma unroll
-        for (int i = 0; i < C::MI; ++i) {
-          const int m = m0 + wm * C::WM + i * 32 + (lane & 31);
-          if (m < p.M && n < rg.N) {
-            const f32x4 v = {acc[j][i][qd * 4], acc[j][i][qd * 4 + 1], acc[j][i][qd * 4 + 2], acc[j][i][qd * 4 + 3]};
-            *reinterpret_cast<f32x4*>(dst + (int64_t)m * rg.N + n) = v;
-          }
+      for (int i = 0; i < C::MI; ++i) {
+        const int m = m0 + wm * C::WM + i * 32 + (lane & 31);
+        if (m < p.M && n < rg.N) {
+          const f32x4 v = {acc[j][i][qd * 4], acc[j][i][qd * 4 + 1], acc[j][i][qd * 4 + 2], acc[j][i][qd * 4 + 3]};
+          *reinterpret_cast<f32x4*>(dst + (int64_t)m * rg.N + n) = v;
         }
       }
     }
-    return;
   }
-  store_tile<C, FP16>(p, rg, m0, n0, acc, lds, wave, lane);
 }
 
 // The tile's outputs: out[m][n..n+3] = round(acc * (sa * sw) + bias[n..n+3]),
@@ -848,8 +684,9 @@ __device__ __forceinline__ void store_tile(const GemmParams& p, const GemmRegion
   }
 }
 
-// One BM x BN output tile with 128 k-bytes per stage (CfgK128).  Layout of a
-// stage in LDS: A rows [BM][128 B], then W rows [BN][128 B]; the 16-byte chunk
+// One BM x BN output tile of region rg; bx counts the region's workgroups.
+// SPLIT: the workgroup sums the 128-k-byte steps of slice `slice` and writes
+// the fp32 sums to p.partial instead of the outputs.  Layout of a stage in LDS: A rows [BM][128 B], then W rows [BN][128 B]; the 16-byte chunk
 // c of row r sits at physical chunk c ^ swz8(r), swz8(r) = (r >> 1) & 7: a
 // fragment read (16 lanes on 16 consecutive rows, one chunk each) then
 // touches all 64 banks once, and a 1 KiB copy (8 rows x 8 chunks) writes one
@@ -862,18 +699,13 @@ __device__ __forceinline__ void store_tile(const GemmParams& p, const GemmRegion
 //      barrier's LDS fence waits for those reads), then the rest, with the
 //      reads of the next stage's first half and the copies of the stage after
 //      next (into this stage's memory) spread between them.
-// Interleaved on one box against the 64-byte form (4 stages, a barrier per
-// MFMA k-step): 4352 x 9216 x 3072 103.8 against 110.0 us, 4352 x 12288 x 3072
-// 137.2 / 146.0, 4352 x 3072 x 12288 120.8 / 127.7, 4096 x 4096 x 12288
-// 137.1 / 151.1; with B's copies after its second half of MFMAs only (as the
-// 64-byte form places them) the gain was 0-5%, and spreading them in the
-// 64-byte form changed nothing.  Two of B's MFMAs ahead of the barrier: 0.7-5%
-// faster again (1536 x 4096 x 12288 77.5 against 81.5 us, 4352 x 3072 x 12288
-// 119.8 / 121.8), one or four: no better.
-template <class C, bool FP16>
-__device__ __forceinline__ void gemm_tile_k128(const GemmParams& p, const GemmRegion& rg, const int bx,
-                                               unsigned char* lds) {
-  static_assert(C::KB == 128 && C::NS == 2, "two stages of 128 k-bytes");
+// Two of B's MFMAs go ahead of the barrier (at 256 x 256 0.7-5% faster than
+// none: 1536 x 4096 x 12288 77.5 against 81.5 us; one or four: no better), and
+// B's copies are spread over its MFMAs (placed after the second half of them,
+// they landed late: 0-5% slower).
+template <class C, bool FP16, bool SPLIT = false>
+__device__ __forceinline__ void gemm_tile(const GemmParams& p, const GemmRegion& rg, const int bx,
+                                               unsigned char* lds, const int slice = 0) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: copy targets go to SGPRs
@@ -898,24 +730,29 @@ __device__ __forceinline__ void gemm_tile_k128(const GemmParams& p, const GemmRe
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)lds;
   const unsigned char* abase = p.a + (int64_t)m0 * p.lda;
   const unsigned char* wbase = rg.w + (int64_t)n0 * p.ldw;
-  const int nk = (p.K + C::KB - 1) / C::KB;
+  const int nkall = (p.K + C::KB - 1) / C::KB;
+  const int kb = SPLIT ? (int)((int64_t)nkall * slice / p.ksplit) : 0;
+  const int nk = SPLIT ? (int)((int64_t)nkall * (slice + 1) / p.ksplit) : nkall;  // end of the steps
 
-  // copy state of one step, as in gemm_tile: past the end of K a lane's chunk
-  // gets the top offset bit (it lands as zeros), and a step at or past the
-  // end gets empty resources, so every step issues the same copies
+  // copy state of one step: the stage's LDS address and the two buffer
+  // resources; past the end of K a lane's chunk would read the next row, so
+  // its offset gets the top bit (out of range: it lands as zeros).  A step at
+  // or past the end (kt >= nk) gets empty resources: its copies fetch nothing
+  // and write zeros into a stage that no later step reads, so every step
+  // issues the same copies and the vmcnt waits stay uniform.
   struct StepCopies {
     u32x4 ra, rw;
     uint32_t st;
-    uint32_t dead;
+    uint32_t dead;  // 0, or 0x80000000 for a lane whose chunk lies past K
   };
-  auto prepare = [&](const int kt) __attribute__((always_inline)) {
+  auto prepare = [&](const int kt, const int stage) __attribute__((always_inline)) {
     StepCopies sc;
     const int koff = kt * C::KB;
     const int lim = p.K - koff;
     const int kin = min(C::KB, lim);
     sc.ra = rsrc_words(abase + koff, kt < nk ? (uint32_t)((mrows - 1) * p.lda + kin) : 0u);
     sc.rw = rsrc_words(wbase + koff, kt < nk ? (uint32_t)((nrows - 1) * p.ldw + kin) : 0u);
-    sc.st = lds0 + (uint32_t)((kt & 1) * C::STAGE);
+    sc.st = lds0 + (uint32_t)(stage * C::STAGE);
     sc.dead = (lim < C::KB && cchunk >= lim) ? 0x80000000u : 0u;
     return sc;
   };
@@ -935,10 +772,10 @@ __device__ __forceinline__ void gemm_tile_k128(const GemmParams& p, const GemmRe
     for (int e = 0; e < 2; ++e)
       fo[h][e] = (uint32_t)(frow * C::KB + ((4 * h + 2 * (lane >> 5) + e) ^ ((frow >> 1) & 7)) * 16);
   constexpr int NRD = 2 * (C::MI + C::NJ);
-  // half r % 2 of fragment r / 2 (A fragments first, then W), k-half h of stage kt
-  auto read_frag = [&](const int kt, const int h, const int r, i32x8 (&fa)[C::MI], i32x8 (&fw)[C::NJ])
+  // half r % 2 of fragment r / 2 (A fragments first, then W), k-half h of a stage
+  auto read_frag = [&](const int stage, const int h, const int r, i32x8 (&fa)[C::MI], i32x8 (&fw)[C::NJ])
       __attribute__((always_inline)) {
-    const unsigned char* st = lds + (kt & 1) * C::STAGE;
+    const unsigned char* st = lds + stage * C::STAGE;
     const int f = r >> 1;
     const unsigned char* b = f < C::MI ? st + (wm * C::WM + f * 32) * C::KB
                                        : st + C::A_BYTES + (wn * C::WN + (f - C::MI) * 32) * C::KB;
@@ -957,34 +794,34 @@ __device__ __forceinline__ void gemm_tile_k128(const GemmParams& p, const GemmRe
 #pragma unroll
     for (int i = 0; i < C::MI; ++i) acc[j][i] = f32x16{};
 
-  // prologue: both stages in flight, stage 0 published, its first half read
-  {
-    const StepCopies s0 = prepare(0);
+  // prologue: every stage in flight, stage 0 published, its first half read
 #pragma unroll
-    for (int c = 0; c < C::COPIES; ++c) issue(s0, c);
-    const StepCopies s1 = prepare(1);
+  for (int s0 = 0; s0 < C::NS; ++s0) {
+    const StepCopies sc = prepare(kb + s0, s0);
 #pragma unroll
-    for (int c = 0; c < C::COPIES; ++c) issue(s1, c);
+    for (int c = 0; c < C::COPIES; ++c) issue(sc, c);
   }
-  wait_vmcnt<C::COPIES>();
+  wait_vmcnt<(C::NS - 1) * C::COPIES>();
   __syncthreads();
   i32x8 fa[2][C::MI], fw[2][C::NJ];
 #pragma unroll
   for (int r = 0; r < NRD; ++r) read_frag(0, 0, r, fa[0], fw[0]);
 
-  // One MFMA k-step on fragments `cur`, with the reads of (stage rkt, half rh)
+  // One MFMA k-step on fragments `cur`, with the reads of (stage rst, half rh)
   // into the other fragments between its MFMAs.  The second k-step (COPY)
   // issues its first PRE MFMAs (their fragments are in registers) before the
   // wait for the next stage's copies and the barrier, so the matrix core has
   // work while the wave waits there; its reads and the copies of sc follow,
   // spread over the remaining MFMAs.
   constexpr int NMF = C::NJ * C::MI;
-  constexpr int PRE = 2 < NMF ? 2 : NMF - 1;
-  auto kstep = [&](auto copy_tag, const int cur, const int rkt, const int rh, const StepCopies& sc)
+  constexpr int PRE = 2 < NMF ? 2 : 1;
+  auto kstep = [&](auto copy_tag, const int cur, const int rst, const int rh, const StepCopies& sc)
       __attribute__((always_inline)) {
     constexpr bool COPY = decltype(copy_tag)::value;
-    constexpr int R0 = COPY ? PRE : 0;  // reads (and copies) after MFMAs [R0, R0 + H)
-    constexpr int H = COPY ? NMF - PRE : (NMF >= 2 ? NMF / 2 : 1);
+    // reads (and copies) after MFMAs [R0, R0 + H); a wave with one MFMA per
+    // k-step (64 x 64 tiles) issues them all after it, behind the barrier
+    constexpr int R0 = COPY ? (NMF > PRE ? PRE : PRE - 1) : 0;
+    constexpr int H = COPY ? NMF - R0 : (NMF >= 2 ? NMF / 2 : 1);
 #pragma unroll
     for (int idx = 0; idx < NMF; ++idx) {
       const int j = idx / C::MI, i = idx % C::MI;
@@ -993,7 +830,7 @@ __device__ __forceinline__ void gemm_tile_k128(const GemmParams& p, const GemmRe
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (COPY) {
         if (idx == PRE - 1) {
-          wait_vmcnt<0>();  // the next stage's copies (issued one step ago) have landed
+          wait_vmcnt<(C::NS - 2) * C::COPIES>();  // the next stage's copies have landed
           __syncthreads();
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -1001,7 +838,7 @@ __device__ __forceinline__ void gemm_tile_k128(const GemmParams& p, const GemmRe
       if (idx >= R0 && idx < R0 + H) {
 #pragma unroll
         for (int r = (idx - R0) * NRD / H; r < (idx - R0 + 1) * NRD / H; ++r)
-          read_frag(rkt, rh, r, fa[cur ^ 1], fw[cur ^ 1]);
+          read_frag(rst, rh, r, fa[cur ^ 1], fw[cur ^ 1]);
         if constexpr (COPY) {
 #pragma unroll
           for (int c = (idx - R0) * C::COPIES / H; c < (idx - R0 + 1) * C::COPIES / H; ++c) issue(sc, c);
@@ -1010,23 +847,23 @@ __device__ __forceinline__ void gemm_tile_k128(const GemmParams& p, const GemmRe
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  for (int kt = 0; kt < nk; ++kt) {
+  int st = 0;  // stage of step kt
+  for (int kt = kb; kt < nk; ++kt) {
     const StepCopies none = {};
-    kstep(std::false_type{}, 0, kt, 1, none);
+    const int nst = st + 1 == C::NS ? 0 : st + 1;
+    kstep(std::false_type{}, 0, st, 1, none);
     __builtin_amdgcn_sched_barrier(0);
-    const StepCopies sc = prepare(kt + 2);
-    kstep(std::true_type{}, 1, kt + 1, 0, sc);
+    const StepCopies sc = prepare(kt + C::NS, st);
+    kstep(std::true_type{}, 1, nst, 0, sc);
+    st = nst;
   }
 
   wait_vmcnt<0>();  // the copies of the steps past the end still land in their stages
+  if constexpr (SPLIT) {
+    store_partial<C>(p, rg, m0, n0, acc, slice, wave, lane);
+    return;
+  }
   store_tile<C, FP16>(p, rg, m0, n0, acc, lds, wave, lane);
-}
-
-// A tile of either form.
-template <class C, bool FP16>
-__device__ __forceinline__ void run_tile(const GemmParams& p, const GemmRegion& rg, const int bx, unsigned char* lds) {
-  if constexpr (C::KB == 128) gemm_tile_k128<C, FP16>(p, rg, bx, lds);
-  else gemm_tile<C, FP16>(p, rg, bx, lds);
 }
 
 // Region 0 (C1 tiles) and region 1 (C2 tiles), one after the other in
@@ -1045,8 +882,8 @@ fp8_gemm_kernel(const GemmParams p) {
   const int bx = blockIdx.x;
   const int off0 = p.small_first ? p.r[1].wgs : 0;  // first workgroup of each region
   const int off1 = p.small_first ? 0 : p.r[0].wgs;
-  if (bx >= off0 && bx < off0 + p.r[0].wgs) run_tile<C1, FP16>(p, p.r[0], bx - off0, lds);
-  else run_tile<C2, FP16>(p, p.r[1], bx - off1, lds);
+  if (bx >= off0 && bx < off0 + p.r[0].wgs) gemm_tile<C1, FP16>(p, p.r[0], bx - off0, lds);
+  else gemm_tile<C2, FP16>(p, p.r[1], bx - off1, lds);
 }
 
 // Split launch: workgroup b sums k-slice b / wgs of tile b % wgs of region 0
@@ -1231,53 +1068,47 @@ int launch_quant(const qik_fp8_quant_args* a, unsigned* ws, hipStream_t s) {
   return hipLaunchKernel(fn, dim3((unsigned)grid), dim3(QT), args, 0, s) == hipSuccess ? QIK_OK : QIK_ERR_LAUNCH;
 }
 
-// GEMM tile shapes, largest first
-// The 256-row pair: 128 k-bytes per stage (CfgK128) and 8 waves, two per
-// SIMD (2 x 4 waves, 128 x 64 wave tiles, 128 accumulators and 240 registers
-// per wave).  With 64 k-bytes per stage, 8 waves against 4 of 128 x 128:
-// 4352 x 9216 x 3072 109.4 against 113.1 us, 4352 x 12288 x 3072 145.8 /
-// 150.6, 4352 x 3072 x 12288 128.7 / 129.3 (interleaved on one box); with 128,
-// 4 waves were within 2% of 8 either way.
-typedef CfgK128<256, 256, 2, 4> Cfg256x256;
-typedef CfgK128<256, 128, 2, 4> Cfg256x128w8;
-typedef Cfg<256, 128, 4> Cfg256x128;
-// The smaller tiles' k-steps are short (four and one MFMAs per wave), so they
-// keep more stages in flight to cover the copies' latency: at 256 x 3072 x
-// 12288 (64 x 64 tiles) 8 stages took 27.9 us against 45.5 with 4 (16: 28.9);
-// at 256 x 9216 x 3072 (128 x 128) 6 stages 17.0 against 18.8 with 4.
-typedef Cfg<128, 128, 6> Cfg128x128;
-typedef Cfg<64, 64, 8> Cfg64x64;
-// The 192-row pair (the reference test's 1536 x 4096 x 4096 takes 256 of its
-// tiles) at 128 k-bytes per stage, 4 waves: 1536 x 4096 x 4096 30.2-31.9
-// against 31.2-33.8 us, 1536 x 4096 x 12288 82.4 / 86.0, interleaved on one
-// box.  The 256 x 128 / 128 x 128 pair stays at 64 k-bytes: at 128 (4 waves,
-// eight MFMAs per step) 768 x 3072 x 12288 took 67.7 against 54.4 us.
-typedef CfgK128<192, 128, 2, 2> Cfg192x128k;
-typedef CfgK128<128, 128, 2, 2> Cfg128x128k;
+// GEMM tile shapes: 8 waves (two per SIMD) down to 128 x 128, 4 waves below
+// (at 4352 rows the 256 x 256 tile of 8 waves was 3% ahead of 4; 192 x 128
+// with 8 waves against 4: 69.7 / 74.3 us at 1728 x 3072 x 12288).
+typedef CfgK128<256, 256, 2, 4, 2> Cfg256x256;
+typedef CfgK128<192, 256, 2, 4, 2> Cfg192x256;
+typedef CfgK128<256, 128, 2, 4, 3> Cfg256x128;
+typedef CfgK128<128, 256, 2, 4, 3> Cfg128x256;
+typedef CfgK128<192, 128, 2, 4, 3> Cfg192x128;
+typedef CfgK128<128, 128, 2, 4, 3> Cfg128x128;
+typedef CfgK128<64, 128, 1, 4, 3> Cfg64x128;
+typedef CfgK128<64, 64, 2, 2, 4> Cfg64x64;
 
-// Time of a tile of each shape relative to a 256 x 256 tile: area / rate,
-// the rates measured on MI355X with each shape forced over whole launches
-// (1536x4096x4096 50.0 / 35.1 / 45.8 us, 4352x9216x3072 146.7 / 153.1 /
-// 201.1 us, 4352x3072x12288 141.4 / 188.0 / 265.1 us for 256x256 / 256x128 /
-// 128x128).  A 256 x 128 tile moves 24 KiB into LDS per 512 MFMA cycles,
-// close to what the copy path sustains, so it runs at about 0.8 of the big
-// tile's rate per output, and 128 x 128 at about 0.6.  The 64 x 64 tile (one
-// MFMA per wave and step) is for launches with few tiles: at 256 x 3072 x
-// 12288 its 192 tiles took 45.7 us against 65.5 for 48 tiles of 128 x 128;
-// 0.3 is the rate that keeps it out of the 512- and 1024-row shapes (0.45
-// chose it there, 16-25% slower).  The 192 x 128 tile makes 256 tiles of
-// 1536 x 4096 (one per CU): 33.0 us against 35.6 for 192 tiles of 256 x 128,
-// a rate of about 0.65.
+// Time of a tile of each shape on a full chip, in us: t0 (prologue, output,
+// the launch's share) + t1 per 128-k-byte step.  Fitted to launches of one
+// round on MI355X, each shape forced (M x N x K 1728 x 9216 x 3072 43.9 us and
+// 4352 x 3072 x 12288 149.5 for 256 x 256; 1152 x 9216 x 3072 33.2, 3456 x
+// 3072 x 12288 135.5 for 192 x 256; 768 x 9216 x 3072 25.0, 1728 x 3072 x
+// 12288 81.2 for 256 x 128; 2600 x 3072 x 3072 27.3, x 12288 87.3 for 128 x
+// 256; 1728 x 3072 x 3072 20.7, x 12288 69.7 for 192 x 128; 1152 x 3072 x 3072
+// 16.4, x 12288 51.7 for 128 x 128; 400 x 3072 x 3072 11.5, x 4096 x 4096 14.1
+// for 64 x 128; 203 x 3072 x 3072 8.9, x 4096 x 4096 11.1 for 64 x 64).  Over
+// 37 shapes of 64 to 4352 rows the plan they give was the fastest single shape
+// measured, or a mix, at every one.
 struct TileShape {
   int bm, bn;
-  double t;
+  double t0, t1;
 };
-static const TileShape kShapes[5] = {
-    {256, 256, 1.0}, {256, 128, 0.5 / 0.8}, {128, 128, 0.25 / 0.6}, {64, 64, 0.0625 / 0.3}, {192, 128, 0.375 / 0.65}};
+enum { T256x256, T256x128, T128x128, T192x128, T192x256, T128x256, T64x128, T64x64, NSHAPES };
+static const TileShape kShapes[NSHAPES] = {{256, 256, 6.0, 1.5},   {256, 128, 6.0, 0.775}, {128, 128, 4.6, 0.485},
+                                           {192, 128, 4.6, 0.67},  {192, 256, 3.5, 1.3},   {128, 256, 6.0, 0.81},
+                                           {64, 128, 3.8, 0.32},   {64, 64, 3.8, 0.215}};
 // the (big, small) shape pairs a launch can take, as indices into kShapes
-static const int kPairs[4][2] = {{0, 1}, {1, 2}, {4, 2}, {2, 3}};
+// (both of a pair have the same number of waves)
+constexpr int NPAIRS = 6;
+static const int kPairs[NPAIRS][2] = {{T256x256, T256x128}, {T256x128, T128x128}, {T192x128, T128x128},
+                                      {T192x256, T192x128}, {T128x256, T128x128}, {T64x128, T64x64}};
+
+inline double tile_time(int shape, int64_t steps) { return kShapes[shape].t0 + kShapes[shape].t1 * (double)steps; }
 
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+inline int64_t steps_of(int64_t K) { return cdiv(K, 128); }  // 128-k-byte steps
 
 // Finish time of one XCD whose P CUs run t1 tiles of time d1 and then t2
 // tiles of time d2, one workgroup per CU (a 256-thread workgroup of these
@@ -1307,11 +1138,11 @@ double xcd_makespan(int64_t t1, double d1, int64_t t2, double d2, int64_t P) {
   return std::max(end1, last + d2);
 }
 
-// Columns [0, n1) with tile shape `big`, [n1, N) with shape big + 1.
+// Columns [0, n1) with the pair's first tile shape, [n1, N) with its second.
 struct GemmPlan {
   int pair;  // index into kPairs
   int64_t n1;
-  double t;  // estimated makespan, in 256 x 256 tile times
+  double t;  // estimated makespan, us
   bool small_first;  // launch the small tiles' region first (fp8_gemm_kernel)
 };
 
@@ -1319,20 +1150,22 @@ struct GemmPlan {
 // to the XCDs in turn, so the XCD that finishes last holds ceil(tiles / 8) of
 // each region.  The split points are whole big-tile columns; n1 = N is one
 // region of the big shape, n1 = 0 one of the small shape.  A later candidate
-// replaces an earlier one only if it is estimated 3% faster (the rates above
+// replaces an earlier one only if it is estimated 3% faster (the times above
 // are good to a few percent); the first candidate is 256 x 256 tiles.
-GemmPlan choose_plan(int64_t M, int64_t N, int cus) {
+GemmPlan choose_plan(int64_t M, int64_t N, int64_t K, int cus) {
   const int64_t P = std::max(1, (cus > 0 ? cus : 256) / 8);
   GemmPlan best = {0, N, 0.0};
   double best_t = 1e300;
-  for (int pr = 0; pr < 4; ++pr) {
+  const int64_t steps = steps_of(K);
+  for (int pr = 0; pr < NPAIRS; ++pr) {
     const TileShape& s1 = kShapes[kPairs[pr][0]];
     const TileShape& s2 = kShapes[kPairs[pr][1]];
+    const double d1 = tile_time(kPairs[pr][0], steps), d2 = tile_time(kPairs[pr][1], steps);
     for (int64_t k = cdiv(N, s1.bn); k >= 0; --k) {
       const int64_t n1 = std::min(k * s1.bn, N);
       const int64_t t1 = cdiv(M, s1.bm) * cdiv(n1, s1.bn);
       const int64_t t2 = cdiv(M, s2.bm) * cdiv(N - n1, s2.bn);
-      const double t = xcd_makespan(cdiv(t1, 8), s1.t, cdiv(t2, 8), s2.t, P);
+      const double t = xcd_makespan(cdiv(t1, 8), d1, cdiv(t2, 8), d2, P);
       if (t < best_t * 0.97) {
         best_t = t;
         best = {pr, n1, t, false};
@@ -1348,27 +1181,32 @@ GemmPlan choose_plan(int64_t M, int64_t N, int cus) {
   const int64_t t1 = cdiv(M, s1.bm) * cdiv(best.n1, s1.bn);
   const int64_t t2 = cdiv(M, s2.bm) * cdiv(N - best.n1, s2.bn);
   if (t1 > 0 && t2 > 0)
-    best.small_first = xcd_makespan(cdiv(t2, 8), s2.t, cdiv(t1, 8), s1.t, P) <= best_t * 1.0001;
+    best.small_first = xcd_makespan(cdiv(t2, 8), tile_time(kPairs[best.pair][1], steps), cdiv(t1, 8),
+                                    tile_time(kPairs[best.pair][0], steps), P) <= best_t * 1.0001;
   return best;
 }
 
-// K-split of a launch with few tiles and many k-steps: S slices of 128 x 128
-// tiles, each summing nk / S k-steps into fp32 partials that a second launch
-// adds in slice order.  Only when it is estimated well ahead of the unsplit
-// plan (the partials, the second launch and the shorter pipelines cost
-// something): at least 96 k-steps, at most half the CUs' worth of tiles.
-// 1 means no split.
-int choose_ksplit(int64_t M, int64_t N, int64_t K, int cus) {
+// K-split of a launch with few tiles and a long K: S slices, each summing its
+// share of the steps into fp32 partials that a second launch adds in slice
+// order.  64 x 64 tiles for at most 64 rows (64 x 3072 x 12288 13.2 us in 4 or
+// 5 slices against 15.9 in 8 slices of 128 x 128), 128 x 128 above.  At least
+// 48 steps, at most half the CUs' worth of tiles, and only when it is
+// estimated ahead of the unsplit plan with the second launch counted (about
+// 2.5 us, and the partials at about 5 TB/s).  slices = 1 means no split.
+struct KSplit {
+  int slices, shape;
+};
+KSplit choose_ksplit(int64_t M, int64_t N, int64_t K, int cus) {
   if (cus <= 0) cus = 256;
-  const int64_t nk = cdiv(K, KB);
-  if (nk < 96) return 1;
-  const int64_t t128 = cdiv(M, 128) * cdiv(N, 128);
-  if (t128 * 2 > cus) return 1;
-  const int S = (int)std::min<int64_t>({cus / t128, 8, nk / 16});
-  if (S < 2) return 1;
-  const int64_t P = std::max(1, cus / 8);
-  const double t_split = xcd_makespan(cdiv(t128 * S, 8), kShapes[2].t / S, 0, 0.0, P);
-  return t_split < 0.6 * choose_plan(M, N, cus).t ? S : 1;
+  const int shape = M <= 64 ? T64x64 : T128x128;
+  const int64_t steps = steps_of(K);
+  if (steps < 48) return {1, shape};
+  const int64_t tiles = cdiv(M, kShapes[shape].bm) * cdiv(N, kShapes[shape].bn);
+  if (tiles * 2 > cus) return {1, shape};
+  const int S = (int)std::min<int64_t>({cus / tiles, 8, steps / 8});
+  if (S < 2) return {1, shape};
+  const double t_split = tile_time(shape, cdiv(steps, S)) + 2.5 + (double)(S * M * N) * 4.0 / 5e6;
+  return {t_split < 0.95 * choose_plan(M, N, K, cus).t ? S : 1, shape};
 }
 
 // tile rows per group of the tile order: the group size that minimises the
@@ -1415,6 +1253,17 @@ int launch_gemm(GemmParams& p, const qik_fp8_gemm_args* a, int64_t n1, bool fp16
   void* args[] = {&p};
   const void* fn = fp16 ? (const void*)fp8_gemm_kernel<C1, C2, true> : (const void*)fp8_gemm_kernel<C1, C2, false>;
   return hipLaunchKernel(fn, dim3(grid), dim3(C1::NT), args, 0, s) == hipSuccess ? QIK_OK : QIK_ERR_LAUNCH;
+}
+
+// The slices' launch of a K split (p.ksplit and p.partial set).
+template <class C>
+int launch_split(GemmParams& p, const qik_fp8_gemm_args* a, bool fp16, hipStream_t s) {
+  if (set_region<C>(p.r[0], a, 0, a->N) != QIK_OK) return QIK_ERR_SHAPE;
+  const int64_t grid = (int64_t)p.r[0].wgs * p.ksplit;
+  if (grid > (int64_t)INT_MAX || (a->M * (a->N / 8) + 255) / 256 > (int64_t)INT_MAX) return QIK_ERR_SHAPE;
+  void* args[] = {&p};
+  const void* fk = fp16 ? (const void*)fp8_gemm_split_kernel<C, true> : (const void*)fp8_gemm_split_kernel<C, false>;
+  return hipLaunchKernel(fk, dim3((unsigned)grid), dim3(C::NT), args, 0, s) == hipSuccess ? QIK_OK : QIK_ERR_LAUNCH;
 }
 
 // ---------------------------------------------------------------------------
@@ -1590,13 +1439,15 @@ int qik_fp8_gemm(const qik_fp8_gemm_args* a, void* stream) {
   p.ldc = a->ldc;
   const bool fp16 = a->out_dtype == QIK_DTYPE_FP16;
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  const GemmPlan plan = choose_plan(a->M, a->N, device_cus());
+  const GemmPlan plan = choose_plan(a->M, a->N, a->K, device_cus());
   p.small_first = plan.small_first ? 1 : 0;
   switch (plan.pair) {
-    case 0: return launch_gemm<Cfg256x256, Cfg256x128w8>(p, a, plan.n1, fp16, s);
+    case 0: return launch_gemm<Cfg256x256, Cfg256x128>(p, a, plan.n1, fp16, s);
     case 1: return launch_gemm<Cfg256x128, Cfg128x128>(p, a, plan.n1, fp16, s);
-    case 2: return launch_gemm<Cfg192x128k, Cfg128x128k>(p, a, plan.n1, fp16, s);
-    default: return launch_gemm<Cfg128x128, Cfg64x64>(p, a, plan.n1, fp16, s);
+    case 2: return launch_gemm<Cfg192x128, Cfg128x128>(p, a, plan.n1, fp16, s);
+    case 3: return launch_gemm<Cfg192x256, Cfg192x128>(p, a, plan.n1, fp16, s);
+    case 4: return launch_gemm<Cfg128x256, Cfg128x128>(p, a, plan.n1, fp16, s);
+    default: return launch_gemm<Cfg64x128, Cfg64x64>(p, a, plan.n1, fp16, s);
   }
 }
 
@@ -1606,7 +1457,7 @@ int qik_fp8_gemm_workspace_size(const qik_fp8_gemm_args* a, int64_t* bytes) {
   *bytes = 0;
   const int st = qik_fp8_gemm_validate(a);
   if (st != QIK_OK) return st;
-  const int S = choose_ksplit(a->M, a->N, a->K, device_cus());
+  const int S = choose_ksplit(a->M, a->N, a->K, device_cus()).slices;
   if (S > 1) *bytes = (int64_t)S * a->M * a->N * (int64_t)sizeof(float);
   return QIK_OK;
 }
@@ -1615,7 +1466,8 @@ int qik_fp8_gemm_ws(const qik_fp8_gemm_args* a, void* workspace, int64_t workspa
   using namespace qik_fp8;
   const int st = qik_fp8_gemm_validate(a);
   if (st != QIK_OK) return st;
-  const int S = choose_ksplit(a->M, a->N, a->K, device_cus());
+  const KSplit ks = choose_ksplit(a->M, a->N, a->K, device_cus());
+  const int S = ks.slices;
   if (S <= 1) return qik_fp8_gemm(a, stream);
   const int64_t need = (int64_t)S * a->M * a->N * (int64_t)sizeof(float);
   if (workspace == nullptr || workspace_bytes < need || !aligned_to(workspace, 16)) return QIK_ERR_WORKSPACE;
@@ -1631,17 +1483,12 @@ int qik_fp8_gemm_ws(const qik_fp8_gemm_args* a, void* workspace, int64_t workspa
   p.ldc = a->ldc;
   p.ksplit = S;
   p.partial = static_cast<float*>(workspace);
-  if (set_region<Cfg128x128>(p.r[0], a, 0, a->N) != QIK_OK) return QIK_ERR_SHAPE;
-  const int64_t grid = (int64_t)p.r[0].wgs * S;
-  const int64_t rgrid = (a->M * (a->N / 8) + 255) / 256;
-  if (grid > (int64_t)INT_MAX || rgrid > (int64_t)INT_MAX) return QIK_ERR_SHAPE;
   const bool fp16 = a->out_dtype == QIK_DTYPE_FP16;
   const hipStream_t s = static_cast<hipStream_t>(stream);
+  const int sst = ks.shape == T64x64 ? launch_split<Cfg64x64>(p, a, fp16, s) : launch_split<Cfg128x128>(p, a, fp16, s);
+  if (sst != QIK_OK) return sst;
+  const int64_t rgrid = (a->M * (a->N / 8) + 255) / 256;
   void* args[] = {&p};
-  const void* fk = fp16 ? (const void*)fp8_gemm_split_kernel<Cfg128x128, true>
-                        : (const void*)fp8_gemm_split_kernel<Cfg128x128, false>;
-  if (hipLaunchKernel(fk, dim3((unsigned)grid), dim3(Cfg128x128::NT), args, 0, s) != hipSuccess)
-    return QIK_ERR_LAUNCH;
   const void* fr = fp16 ? (const void*)splitk_reduce_kernel<true> : (const void*)splitk_reduce_kernel<false>;
   return hipLaunchKernel(fr, dim3((unsigned)rgrid), dim3(256), args, 0, s) == hipSuccess ? QIK_OK : QIK_ERR_LAUNCH;
 }
@@ -1652,14 +1499,15 @@ int qik_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, int32_t cus, int32_t* pla
   if (M < 1 || N < 16 || K < 16 || N % 16 != 0 || K % 16 != 0) return QIK_ERR_SHAPE;
   if (M > (int64_t)INT_MAX || N > (int64_t)INT_MAX || K > (int64_t)(INT_MAX / 256)) return QIK_ERR_SHAPE;
   if (cus <= 0) cus = 256;
-  const int S = choose_ksplit(M, N, K, cus);
-  if (S > 1) {
-    const int32_t v[6] = {128, 128, 128, 128, 0, S};
+  const KSplit ks = choose_ksplit(M, N, K, cus);
+  if (ks.slices > 1) {
+    const TileShape& sp = kShapes[ks.shape];
+    const int32_t v[6] = {sp.bm, sp.bn, sp.bm, sp.bn, 0, ks.slices};
     memcpy(plan, v, sizeof(v));
     *n1 = N;
     return QIK_OK;
   }
-  const GemmPlan g = choose_plan(M, N, cus);
+  const GemmPlan g = choose_plan(M, N, K, cus);
   const TileShape& s1 = kShapes[kPairs[g.pair][0]];
   const TileShape& s2 = kShapes[kPairs[g.pair][1]];
   const int32_t v[6] = {s1.bm, s1.bn, s2.bm, s2.bn, g.small_first ? 1 : 0, 1};

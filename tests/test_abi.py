@@ -403,6 +403,27 @@ def test_fp8_gemm_plan(mnk, plan, n1):
     assert list(got) == plan and n.value == n1
 
 
+@pytest.mark.parametrize("mnk,plan,n1", [
+    ((17, 2736, 208), [64, 128, 64, 64, 0, 1], 0),
+    ((90, 8352, 192), [64, 128, 64, 64, 0, 1], 8352),
+    ((324, 6032, 160), [256, 128, 128, 128, 0, 1], 0),
+    ((658, 5600, 400), [192, 128, 128, 128, 0, 1], 5600),
+    ((774, 6640, 528), [256, 256, 256, 128, 0, 1], 0),
+    ((1050, 6848, 656), [128, 256, 128, 128, 0, 1], 6848),
+    ((1566, 3680, 160), [192, 256, 192, 128, 0, 1], 3680),
+    ((2075, 7184, 272), [192, 256, 192, 128, 1, 1], 5888),
+    ((40, 1040, 8208), [64, 64, 64, 64, 0, 8], 1040),
+    ((64, 3072, 12288), [64, 64, 64, 64, 0, 5], 3072),
+    ((65, 1040, 8208), [128, 128, 128, 128, 0, 8], 1040),
+])
+def test_fp8_gemm_plan_tile_shapes(mnk, plan, n1):
+    """Every tile shape and both K-split shapes are reached (256 CUs)."""
+    got = (ctypes.c_int32 * 6)()
+    n = ctypes.c_int64()
+    assert _lib.load().qik_fp8_gemm_plan(*mnk, 0, got, ctypes.byref(n)) == 0
+    assert list(got) == plan and n.value == n1
+
+
 def test_fp8_gemm_plan_checks():
     lib = _lib.load()
     got = (ctypes.c_int32 * 6)()

@@ -267,6 +267,31 @@ def test_gemm_vs_fp64_oracle(qik, M, N, K, bias):
     _check_close(out, ref, _abs_sum(xq, wq, sx, sw, bnp))
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (17, 2736, 208),      # 64 x 64 tiles (4 stages), 2 steps: fewer than the stages, a 80-byte tail
+    (64, 1040, 1104),     # 64 x 64 tiles, a whole row block, 9 steps
+    (90, 8352, 192),      # 64 x 128 tiles (3 stages), 2 steps
+    (129, 8352, 528),     # 64 x 128 tiles, one row past two row blocks, 5 steps
+    (324, 6032, 160),     # 128 x 128 tiles (3 stages), 2 steps
+    (658, 5600, 400),     # 192 x 128 tiles (3 stages), 4 steps, 16-byte tail
+    (774, 6640, 528),     # 256 x 128 tiles (3 stages), 5 steps
+    (1050, 6848, 656),    # 128 x 256 tiles (3 stages)
+    (1566, 3680, 160),    # 192 x 256 tiles (2 stages), 2 steps
+    (2075, 7184, 272),    # 192 x 128 then 192 x 256 columns
+    (40, 1040, 8208),     # K split in 8 of 64 x 64 tiles, 65 steps
+    (65, 1040, 8208),     # K split in 8 of 128 x 128 tiles
+])
+def test_gemm_tile_shapes_vs_fp64_oracle(qik, M, N, K):
+    """One shape per tile shape and stage count, at ragged sizes and at step
+    counts below, at and just past the stages in flight."""
+    a, w, xq, wq, sx, sw = _gemm_operands(M, N, K, 2000 + M + N + K)
+    b = torch.randn(N, generator=torch.Generator().manual_seed(10)).to(torch.bfloat16)
+    out = qik.fp8_linear(a, w, torch.tensor([sx], device=DEV), torch.tensor([sw], device=DEV), b.to(DEV))
+    acc = torch.from_numpy(of.decode(xq)).to(DEV).double() @ torch.from_numpy(of.decode(wq)).to(DEV).double().T
+    ref = (acc * float(np.float32(sx * sw)) + b.to(DEV).double()[None, :]).cpu().numpy()
+    _check_close(out, ref, _abs_sum(xq, wq, sx, sw, b.float().numpy()))
+
+
 def test_gemm_fp16_out_and_strided_rows(qik):
     M, N, K = 640, 512, 1024
     a, w, xq, wq, sx, sw = _gemm_operands(M, N, K, 77, lda=1040)
