@@ -120,7 +120,9 @@ int qik_attn_fwd(const qik_attn_args* args, void* stream);
  * arrival counts) and the partial softmax states of split row blocks: the
  * launch runs whole rounds of row blocks, then splits each row block of the
  * last, partly filled round over its KV tiles into two pieces (seven tenths
- * and three tenths of its tiles) that the second to finish combines.  The
+ * and three tenths of its tiles; four or eight equal ones when the round fills
+ * less than a sixth or at most a sixteenth of the device) that the last to
+ * finish combines.  The
  * size depends on the shape and on the device's CU count only,
  * stays below 2 x (workgroups resident at once) x (BM x D x 4 + 2 KiB)
  * + 32 KiB (about 70 MB on MI355X, D = 128), and is about 41 MB for
@@ -171,8 +173,9 @@ int qik_attn_fwd_noalloc(const qik_attn_args* args, void* stream);
  * when item/piece/group are not NULL (cap >= grid entries each), per
  * workgroup (or, for qik_attn_fwd_ws, queue position loc of XCD x at index
  * loc * 8 + x): its row block (-1: no work), its piece and its workspace
- * group (-1: not split).  The second piece of a row block with fewer than 16
- * KV tiles is skipped on the device (the first runs the whole row block).
+ * group (-1: not split).  The other pieces of a row block with few KV tiles
+ * (fewer than 16, four per piece when there are more than two) are skipped on
+ * the device (the first runs the whole row block).
  * `split` = 0 gives qik_attn_fwd's assignment.  This form assumes the 8 XCDs
  * of an MI355X; the launches use the XCD count the device reports. */
 int qik_attn_work_map(int64_t n_items, int32_t n_row_blocks, int32_t slots_per_xcd, int32_t split,

@@ -100,6 +100,19 @@ struct Params {
 // (7 T + 5) / 10 tiles (half of them, (T + 1) / 2, when the plan says `even`)
 // and piece 1 the rest.
 constexpr int SPLIT_MIN_TILES = 16;
+// An item of four or eight pieces (a nearly empty last round, qik_plan.h) is
+// cut into equal ones, and runs whole below four tiles a piece.
+constexpr int MANY_MIN_TILES = 4;
+// The two-group kernel splits more finely: its launches leave most of the
+// device idle, so a piece or a group is worth having wherever it saves more
+// than its merge.  Two groups merge in LDS (about 1 us) from 4 tiles on, two
+// pieces through the workspace (about 4 us) from 8.  Against 16 for both
+// (interleaved, us): 12 row blocks of 5 tiles 12.0 -> 10.8, 27 of 18 tiles 21.7
+// -> 18.1, 78 of 26 26.6 -> 22.5, 128 of 15 27.0 -> 19.6, 16 of 12 20.7 -> 15.2
+// (pieces from 16: 16.5); groups from 2 or 8 tiles: no different, except the
+// 5-tile launch at 8 (12.0).
+constexpr int GROUP_MIN_TILES = 4;
+constexpr int PIECE_MIN_TILES = 8;
 
 // Partial softmax state of one thread of a split piece: its DBLK x 16 fp32
 // O^T accumulators (relative to its row's reference point m) and (m, l share).
@@ -369,6 +382,9 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
   static_assert(BN == 64, "one key_valid byte per lane of wave 0");
 
   static_assert(KSPLIT == 1 || KSPLIT == 2, "one or two groups of waves");
+  // items of more than two pieces: not in the two-group kernel, and not at
+  // D = 256 (max_pieces), whose registers are full
+  constexpr bool MANY = KSPLIT == 1 && D <= 128;
   // per group: K stage 0, K stage 1, V stage 0, V stage 1 (one contiguous block)
   __shared__ u32x4 stg[4 * KSPLIT][TILE_BYTES / 16];
   __shared__ uint32_t skv[KSPLIT][2][BN / 4];   // key_valid bytes of each stage's tile (4 per word)
@@ -572,11 +588,18 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
     auto piece_tiles = [&](int T, int& g0, int& g1) {
       // this unit's tiles [g0, g1): all of them, or one of the item's two
       // pieces (T, and so the split, is the same for both pieces of the item)
-      const bool split = wk.group >= 0 && T >= SPLIT_MIN_TILES;
+      bool split = wk.group >= 0 && T >= (KSPLIT == 1 ? SPLIT_MIN_TILES : PIECE_MIN_TILES);
       if constexpr (KSPLIT == 1) {
-        const int gsplit = p.plan.even ? (T + 1) / 2 : (7 * T + 5) / 10;
-        g0 = (split && wk.piece) ? gsplit : 0;
-        g1 = (split && !wk.piece) ? gsplit : T;
+        const int ns = p.plan.ns;
+        if (MANY && ns > 2) {
+          split = split && T >= MANY_MIN_TILES * ns;
+          g0 = split ? T * wk.piece / ns : 0;
+          g1 = split ? T * (wk.piece + 1) / ns : T;
+        } else {
+          const int gsplit = p.plan.even ? (T + 1) / 2 : (7 * T + 5) / 10;
+          g0 = (split && wk.piece) ? gsplit : 0;
+          g1 = (split && !wk.piece) ? gsplit : T;
+        }
       } else {
         // the workgroup's part of the row block (all of it, or one of two equal
         // halves), split between the groups; group 0's waves are the older ones
@@ -586,7 +609,7 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
         const int h = (T + 1) / 2;
         const int a = (split && wk.piece) ? h : 0;
         const int e = (split && !wk.piece) ? h : T;
-        gsplit_on = e - a >= SPLIT_MIN_TILES;
+        gsplit_on = e - a >= GROUP_MIN_TILES;
         const int mid = a + (9 * (e - a) + 8) / 16;
         g0 = (gsplit_on && grp) ? mid : a;
         g1 = (gsplit_on && !grp) ? mid : e;
@@ -812,9 +835,10 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
     }
 
 
-    // ---- split item: both pieces publish their partial state; the second to
-    // arrive combines the two in piece order (so the result does not depend
-    // on which piece that is) and writes the output.  Nothing waits on another
+    // ---- split item: the pieces publish their partial state; the last to
+    // arrive combines them in piece order (so the result does not depend
+    // on which piece that is) and writes the output (told here for two pieces;
+    // with ns of them the last sees ns - 1 where the second sees 1).  Nothing waits on another
     // workgroup.  Ordering, at agent (device) scope:
     //   * a piece that publishes writes its slot with device-scope stores (sc1: written
     //     through past the XCD's L2), then waits for all of them to complete
@@ -885,7 +909,8 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
       // it back).  A piece that finds the other one already arrived merges
       // at once and never writes its own slot; otherwise it publishes its
       // slot and arrives, and the second to arrive merges.
-      if (lead) sred[0][0] = g_load(word) == 1u ? 1 : 0;
+      const unsigned others = MANY ? (unsigned)(pe.plan.ns - 1) : 1u;
+      if (lead) sred[0][0] = g_load(word) == others ? 1 : 0;
       __syncthreads();
       const bool other_first = sred[0][0] != 0;
       __syncthreads();  // every thread has read the flag before it is reused
@@ -909,7 +934,7 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
         __syncthreads();
         if (lead) {
           const unsigned before = g_fetch_add(word, 1u);
-          const bool last = before == 1u;
+          const bool last = before == others;
           if (last) g_store(word, 0u);
           sred[0][0] = last ? 1 : 0;
         }
@@ -921,7 +946,52 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
       // the other piece's state; the two combine in piece order, the same
       // arithmetic whichever of them arrived last (in the two-group kernel
       // group 0 holds the workgroup's state and stores the rows)
-      if (KSPLIT == 1 || grp == 0) {
+      if (MANY && pe.plan.ns > 2) {
+        // ns pieces: every (m, l) first, then the accumulators piece by piece,
+        // this piece's own in its turn.  Explicit fmas: the compiler takes the
+        // products of its own state out of the loop otherwise, and rounds them
+        // where a loaded piece's are fused, so that the bits would depend on
+        // which piece merges.
+        const int ns = pe.plan.ns;
+        float mm = m_run;
+        for (int pc = 0; pc < ns; ++pc) {
+          if (pc == wk.piece) continue;
+          const auto sl = make_rsrc(gslots + pc * SB, SB);
+          mm = fmaxf(mm, __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(
+                                                       sl, (uint32_t)(OB + tid * 8), 0, SC1))[0]);
+        }
+        l_part = 0.0f;
+        f32x16 macc[DBLK];
+#pragma unroll
+        for (int db = 0; db < DBLK; ++db) macc[db] = f32x16{};
+        for (int pc = 0; pc < ns; ++pc) {
+          if (pc == wk.piece) {
+            const float a = (m_run == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(m_run - mm);
+            l_part = __builtin_fmaf(l_run, a, l_part);
+#pragma unroll
+            for (int db = 0; db < DBLK; ++db)
+#pragma unroll
+              for (int i = 0; i < 16; ++i) macc[db][i] = __builtin_fmaf(oacc[db][i], a, macc[db][i]);
+            continue;
+          }
+          const auto sl = make_rsrc(gslots + pc * SB, SB);
+          const f32x2 ml = __builtin_bit_cast(
+              f32x2, __builtin_amdgcn_raw_buffer_load_b64(sl, (uint32_t)(OB + tid * 8), 0, SC1));
+          f32x4 v[DBLK * 4];
+#pragma unroll
+          for (int i = 0; i < DBLK * 4; ++i)
+            v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                 sl, (uint32_t)((i * NTHREADS + tid) * 16), 0, SC1));
+          const float a = (ml[0] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(ml[0] - mm);
+          l_part = __builtin_fmaf(ml[1], a, l_part);
+#pragma unroll
+          for (int i = 0; i < DBLK * 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) macc[i / 4][4 * (i % 4) + e] = __builtin_fmaf(v[i][e], a, macc[i / 4][4 * (i % 4) + e]);
+        }
+#pragma unroll
+        for (int db = 0; db < DBLK; ++db) oacc[db] = macc[db];
+      } else if (KSPLIT == 1 || grp == 0) {
         const auto other = make_rsrc(gslots + (wk.piece ^ 1) * SB, SB);
         const f32x2 mlo = __builtin_bit_cast(
             f32x2, __builtin_amdgcn_raw_buffer_load_b64(other, (uint32_t)(OB + tid * 8), 0, SC1));
@@ -1233,7 +1303,7 @@ int plan_launch(const qik_attn_args* a, bool split, Launch* L) {
       // of the heads), each row block split into two equal pieces on two CUs,
       // every piece split between the groups, the pieces merged through the
       // workspace as the split launch below merges them
-      L->plan = make_plan((int)n, (int)nmb, cus / nx, 1, (a->flags & QIK_UNIFORM_L) ? 0 : 1, nx);
+      L->plan = make_plan((int)n, (int)nmb, cus / nx, 1, (a->flags & QIK_UNIFORM_L) ? 0 : 1, nx, 2);
       if (L->plan.ns == 2 && L->plan.wpx <= cus / nx && 2 * NXCD_MAX + L->plan.ngroups <= QIK_ATTN_WS_CTL_BYTES / 4) {
         L->grid = (int64_t)nx * L->plan.wpx;
         L->ctl_bytes = QIK_ATTN_WS_CTL_BYTES;
@@ -1248,7 +1318,7 @@ int plan_launch(const qik_attn_args* a, bool split, Launch* L) {
   if (split) {
     const int st = slots_per_xcd(L->fn, pick_index((int)a->D, fp16, vfp8, kv), &sx);
     if (st != QIK_OK) return st;
-    L->plan = make_plan((int)n, (int)nmb, sx, 1, (a->flags & QIK_UNIFORM_L) ? 0 : 1, nx);
+    L->plan = make_plan((int)n, (int)nmb, sx, 1, (a->flags & QIK_UNIFORM_L) ? 0 : 1, nx, a->D <= 128 ? MAX_PIECES : 2);
     // queue positions are mapped through loc * nx + x, which must fit an
     // int, and the arrival words must fit the fixed control region (the same
     // for every shape, so that no launch leaves slot data where another

@@ -13,8 +13,9 @@
 //
 // An XCD holds `sx` workgroups at once.  Items that fill whole rounds of sx
 // run as one unit each; each item of the last, partly filled round is split
-// over its KV tiles into two pieces: a big one (the first seven tenths of its
-// tiles) and a small one (the rest).  The order lists the big pieces of all
+// over its KV tiles into pieces.  Usually two: a big one (the first seven
+// tenths of its tiles) and a small one (the rest); four or eight equal ones when
+// the round is nearly empty (plan_pieces).  The order lists the big pieces of all
 // left-over items first, then the small ones.  The launch with a workspace
 // runs sx workgroups per XCD that pull the XCD's units from a queue in this
 // order.  The two workgroups of a CU progress at different rates (the older
@@ -25,7 +26,7 @@
 // the early slot idle while the late one finishes.  When an XCD has no whole
 // round and every piece gets a slot of its own (a launch smaller than the
 // device), all pieces start together and the launch lasts as long as the
-// biggest: then the pieces are equal halves.  The two pieces of an item combine
+// biggest: then the pieces are equal halves.  The pieces of an item combine
 // their partial softmax states through the workspace slots of its group.
 //
 // plan_work(pl, loc * nx + x) is the unit at queue position loc of XCD x;
@@ -45,7 +46,7 @@ namespace qik {
 
 constexpr int NXCD = 8;        // XCDs of an MI355X (the plan's default)
 constexpr int NXCD_MAX = 32;   // largest XCD count a plan takes (control-word layout)
-constexpr int MAX_PIECES = 2;
+constexpr int MAX_PIECES = 8;
 
 struct WorkPlan {
   int nx;                // XCDs the workgroups are dealt to (1 .. NXCD_MAX)
@@ -70,8 +71,21 @@ struct Work {
 // Items of an XCD with q items that run whole when it holds sx workgroups.
 QIK_HD inline int plan_full(int q, int sx) { return q >= sx ? sx * (q / sx) : 0; }
 
-// Pieces per split item: two (see above).
-inline int plan_pieces(int r) { return r > 0 ? MAX_PIECES : 1; }
+// Pieces per split item when an XCD of sx slots has r left-over items: two
+// (see above); after at least one whole round, four when they fill less than a
+// sixth of the slots, eight when at most a sixteenth: two pieces would leave
+// the CUs idle for most of a piece's time (2 x 24 heads x 2772 rows against
+// 4907 keys, 4 row blocks of 132 per XCD left over: 394 us with two pieces, 375
+// with four, 371 with eight; 2 x 24 x 2700 against 3500 265 / 257 / 256).  More
+// pieces cost their merge, one slot after the other (about 4 us each), so a
+// fuller round keeps two (four and eight pieces of a half-full round: 351 and
+// 378 us against 345).
+inline int plan_pieces(int r, int sx, bool rounds) {
+  if (r <= 0) return 1;
+  if (rounds && r * 16 <= sx) return MAX_PIECES;
+  if (rounds && r * 6 < sx) return 4;
+  return 2;
+}
 
 // n items, nmb per (b, h); `split` = 0 runs every item whole.  `ragged`: the
 // items of a head differ in weight (per-row causal lengths), so an XCD that
@@ -81,7 +95,8 @@ inline int plan_pieces(int r) { return r > 0 ? MAX_PIECES : 1; }
 // blocks while at most two heads' K/V are in flight in its L2 (measured on
 // MI355X: three heads rank-major fetch 1.4x the bytes at the same time, one
 // head at a time is 8% slower); with equal items it keeps them head-major.
-inline WorkPlan make_plan(int n, int nmb, int sx, int split, int ragged = 1, int nx = NXCD) {
+inline WorkPlan make_plan(int n, int nmb, int sx, int split, int ragged = 1, int nx = NXCD,
+                          int max_pieces = MAX_PIECES) {
   WorkPlan pl;
   if (nx < 1) nx = 1;
   if (nx > NXCD_MAX) nx = NXCD_MAX;
@@ -99,7 +114,7 @@ inline WorkPlan make_plan(int n, int nmb, int sx, int split, int ragged = 1, int
   }
   const int r_lo = pl.per - pl.full_lo, r_hi = pl.per + 1 - pl.full_hi;
   const int r_max = (pl.rem > 0 && r_hi > r_lo) ? r_hi : r_lo;
-  pl.ns = plan_pieces(r_max);
+  pl.ns = split ? plan_pieces(r_max, sx, pl.full_lo > 0 && max_pieces > 2) : 1;
   const int w_lo = pl.full_lo + pl.ns * r_lo;
   const int w_hi = pl.rem > 0 ? pl.full_hi + pl.ns * r_hi : 0;
   pl.wpx = w_lo > w_hi ? w_lo : w_hi;

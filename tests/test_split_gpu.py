@@ -211,6 +211,71 @@ def test_split_decode_against_fp8_slab(H):
     _check(out, ref, "fp8 slab decode")
 
 
+@pytest.mark.parametrize("H,D,rows,keys,pieces,dtype", [
+    (65, 128, 1024, 2100, 8, torch.bfloat16),   # 65 row blocks per XCD: one left over, 33 tiles in 8 pieces
+    (65, 128, 1024, 2000, 8, torch.bfloat16),   # 32 tiles: the fewest that 8 pieces take
+    (65, 128, 1024, 1970, 8, torch.float16),    # 31 tiles: the left-over row blocks run whole
+    (72, 128, 1000, 1100, 4, torch.bfloat16),   # 72 per XCD: 8 left over, 18 tiles in 4 pieces
+    (97, 64, 1000, 2500, 8, torch.bfloat16),    # D = 64, three workgroups per CU: 97 row blocks on 96 slots
+])
+def test_nearly_empty_last_round(H, D, rows, keys, pieces, dtype):
+    """More row blocks than slots by a few per XCD: the left-over ones run as four or
+    eight pieces merged through the workspace, with rows that see no key in most
+    pieces (short L) or at all (L = -1), and the same bits on every run."""
+    _flush(f"case split last round H={H} D={D} rows={rows} keys={keys}")
+    per = H * -(-rows // 128) // 8
+    sx = (3 if D == 64 else 2) * _cus() // 8
+    grid, ngroups, ns = ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int32()
+    _lib.check(_lib.load().qik_attn_work_map(8 * per, -(-rows // 128), sx, 1, None, None, None, 0, ctypes.byref(grid),
+                                             ctypes.byref(ngroups), ctypes.byref(ns)), "work map")
+    if _cus() == 256:
+        assert ns.value == pieces
+    g = torch.Generator(device=DEV).manual_seed(50 + H + keys)
+    q = torch.randn(1, rows, H, D, generator=g, device=DEV).to(dtype)
+    k, v = (torch.randn(1, keys, H, D, generator=g, device=DEV).to(dtype) for _ in range(2))
+    L = np.full(rows, keys - 1, dtype=np.int32)
+    L[5::17] = np.random.default_rng(keys).integers(-1, keys, size=len(L[5::17]))
+    L[7] = -1
+    Ld = torch.from_numpy(L).to(DEV)
+    outs = [qik.block_causal_flash_attention(q, k, v, Ld, None) for _ in range(3)]
+    for o in outs[1:]:
+        assert torch.equal(outs[0], o)
+    plain = qik.block_causal_flash_attention(q, k, v, Ld, None, split_tail=False)
+    d = (outs[0].float() - plain.float()).abs()
+    assert d.max().item() <= 2 * MAX_ABS and d.mean().item() <= 5e-4
+    heads = [(per * x + per - 1) // -(-rows // 128) for x in (0, 3, 7)]   # heads of left-over row blocks
+    sel = [t[:, :, heads].contiguous().cpu() for t in (q, k, v)]
+    ref = oa.attention_fp32(*sel, L)
+    _check(outs[0][:, :, heads], ref, f"last round H={H}")
+    assert (outs[0][:, 7] == 0).all()
+
+
+@pytest.mark.parametrize("keys", [64, 129, 250, 257, 449, 512, 575, 960, 1000])
+@pytest.mark.parametrize("dtype,v_fp8", [(torch.bfloat16, False), (torch.float16, False), (torch.bfloat16, True)])
+def test_small_launch_groups_and_pieces(keys, dtype, v_fp8):
+    """A launch of few row blocks over 1 to 17 KV tiles: one group, two groups (from 4
+    tiles on), two pieces of one or two groups (from 8 tiles on)."""
+    _flush(f"case small launch keys={keys} {dtype} fp8={v_fp8}")
+    g = torch.Generator().manual_seed(60 + keys)
+    B, H, D, rows = 1, 3, 128, 140
+    P = 70 if v_fp8 else 0
+    q = torch.randn(B, rows, H, D, generator=g).to(dtype)
+    k, v = (torch.randn(B, keys, H, D, generator=g).to(dtype) for _ in range(2))
+    L = np.full(rows, P + keys - 1, dtype=np.int32)
+    L[3::5] = np.random.default_rng(keys).integers(-1, P + keys, size=len(L[3::5]))
+    slab, ref_slab = {}, {}
+    if v_fp8:
+        pk, pv = (torch.randn(B, P, H, D, generator=g).to(dtype) for _ in range(2))
+        cache = qik.ContiguousKVCache(1, B, P + 16, H, D, v_fp8=True, device=DEV)
+        cache.get_layer(0).store(pk.to(DEV), pv.to(DEV))
+        kc, vc, sc = cache.get_layer(0).views()
+        slab = dict(cache_k=kc, cache_v=vc, cache_v_scale=sc)
+        ref_slab = dict(cache_k=kc.cpu(), cache_v=vc.cpu(), cache_v_scale=sc.cpu())
+    out = qik.block_causal_flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), torch.from_numpy(L).to(DEV), None, **slab)
+    ref = oa.attention_fp32(q, k, v, L, None, **ref_slab)
+    _check(out, ref, f"small launch keys={keys}")
+
+
 @pytest.mark.parametrize("name", ["t2i_512", "t2i_512_b2", "t2i_1024_h3"])
 def test_split_is_bit_identical_run_to_run(name):
     """Whichever piece arrives last merges, in piece order: the result never changes."""

@@ -129,6 +129,35 @@ def test_piece_counts_of_the_benchmark_shapes():
     assert work_map(1024, 32, 64, 1)[3:] == (0, 1)
 
 
+@pytest.mark.parametrize("n,nmb,sx,ns", [
+    (1056, 22, 64, 8),   # 2 x 24 heads x 2772 rows: 132 per XCD, 4 left over
+    (520, 8, 64, 8),     # one left over per XCD
+    (513, 9, 64, 8),     # one left over on the first XCD only
+    (576, 24, 64, 4),    # 8 left over
+    (592, 37, 64, 4),    # 10 left over
+    (600, 25, 64, 2),    # 11 left over: more than a sixth
+    (32, 4, 64, 2),      # no whole round
+])
+def test_nearly_empty_last_round_is_cut_finer(n, nmb, sx, ns):
+    """After whole rounds, a few left-over row blocks run as four or eight pieces: every
+    row block once, pieces 0 .. ns-1 of one group, listed piece by piece."""
+    item, piece, group, ngroups, got = work_map(n, nmb, sx, 1)
+    assert got == ns
+    whole, pieces = np.zeros(n, dtype=np.int64), {}
+    for it, pc, gr in zip(item, piece, group):
+        if it >= 0 and gr < 0:
+            whole[it] += 1
+        elif it >= 0:
+            pieces.setdefault(it, []).append((pc, gr))
+    for it, ps in pieces.items():
+        assert sorted(pc for pc, _ in ps) == list(range(ns)) and len({gr for _, gr in ps}) == 1 and whole[it] == 0
+    assert ((whole + np.array([i in pieces for i in range(n)])) == 1).all()
+    assert sorted(ps[0][1] for ps in pieces.values()) == list(range(ngroups))
+    for x in range(NXCD):
+        px = [pc for it, pc, gr in zip(item[x::NXCD], piece[x::NXCD], group[x::NXCD]) if it >= 0 and gr >= 0]
+        assert px == sorted(px)
+
+
 def test_pair_rank_major_order_puts_light_row_blocks_last():
     """24 heads x 34 row blocks: each XCD's run is 3 whole heads, walked rank-major over
     its first two heads (heaviest row block of both first), then the third head
