@@ -112,6 +112,39 @@ def test_quantiser_one_pass_and_two_pass_forms_in_turn(qik):
         del x, got_q, want_q
 
 
+@pytest.mark.parametrize("n,dtype,where", [
+    (28 << 20, torch.float32, 0),            # just past the registers: 1024 blocks of 28 whole steps
+    ((28 << 20) + 1027, torch.float32, -1),  # a ragged last step, elements past the last vector
+    ((57 << 20) + 13, torch.bfloat16, -1),
+    ((57 << 20) + 8 * 1025, torch.float16, 1 << 20),
+])
+@pytest.mark.parametrize("which", ["act", "weight"])
+def test_two_pass_quantiser_edges(qik, n, dtype, where, which):
+    """Sizes past the one-pass form: every code and the scale, as torch's ops give them
+    on the device, with the maximum first, last or inside; bytes past the end kept."""
+    print(f"case two-pass quantiser {n} {dtype} {which}", flush=True)
+    from qwen_image_kernel_amd import _lib
+    from qwen_image_kernel_amd import fp8 as f8
+    import ctypes
+    x = torch.randn(n, generator=torch.Generator(device=DEV).manual_seed(n), device=DEV).to(dtype)
+    x[where] = -37.0
+    out = torch.full((n + 64,), 0x55, dtype=torch.uint8, device=DEV)
+    scale = torch.empty(1, device=DEV)
+    lib = _lib.load()
+    args = f8.quant_args(x, out[:n], scale, _lib.FP8_ACTIVATION if which == "act" else _lib.FP8_WEIGHT)
+    need = ctypes.c_int64(0)
+    assert lib.qik_fp8_quant_workspace_size(ctypes.byref(args), ctypes.byref(need)) == 0
+    ws = torch.zeros(need.value, dtype=torch.uint8, device=DEV)
+    for _ in range(2):
+        assert lib.qik_fp8_quantize(ctypes.byref(args), ws.data_ptr(), need.value,
+                                    torch.cuda.current_stream().cuda_stream) == 0
+    s = (torch.tensor(37.0, device=DEV) * torch.tensor(1.0 / 448.0, device=DEV)).clamp_min(1e-12)
+    y = x.float() * (1.0 / s) if which == "act" else (x.float() / s).clamp(-448.0, 448.0)
+    assert scale.item() == s.item()
+    assert torch.equal(out[:n], y.to(torch.float8_e4m3fn).view(torch.uint8))
+    assert (out[n:] == 0x55).all()
+
+
 @pytest.mark.parametrize("amax", [1.0, 448.0, 3.0, 2.0 ** -20, 2.0 ** 20, 1e-30, 1e30, 1e-13, 5e-10, 7.0, 0.1,
                                   1000.0])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
