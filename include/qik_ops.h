@@ -49,6 +49,13 @@ typedef struct qik_rms_rope_args {
 
 int qik_rms_rope(const qik_rms_rope_args* args, void* stream);
 
+/* Both calls in one launch (a layer's Q and K; no counterpart in the
+ * reference, which launches its kernel once for each): the same results and
+ * the same checks as qik_rms_rope(a) then qik_rms_rope(b), which must have the
+ * same D (QIK_ERR_HEAD_DIM) and dtype (QIK_ERR_DTYPE).  The outputs must not
+ * overlap each other or the other call's x. */
+int qik_rms_rope_pair(const qik_rms_rope_args* a, const qik_rms_rope_args* b, void* stream);
+
 /* One layer's prefix K/V into the slab (layout [B, H, P_max, D] per layer):
  *   k_dst[b, h, p, :] = k[b, p, h, :]
  *   bf16/fp16 V:  v_dst[b, h, p, :] = v[b, p, h, :]

@@ -59,16 +59,7 @@ def fused_rms_norm_rope(
     # checked and prepared once per key -- the argument struct with the
     # weight and cos/sin pointers filled in, the output shape.  Only x's and
     # the output's data pointers change between calls.
-    key = (x.shape, x.stride(), x.data_ptr() & 15, x.dtype, x.device, eps,
-           weight.data_ptr(), weight._version, weight.dtype, weight.shape, weight.stride(), weight.device,
-           freqs_cis.data_ptr(), freqs_cis._version, freqs_cis.dtype, freqs_cis.shape, freqs_cis.stride(),
-           freqs_cis.device)
-    ent = _CALLS.get(key)
-    if ent is None:
-        ent = _prepare(x, weight, freqs_cis, eps)
-        if len(_CALLS) >= 64:
-            _CALLS.clear()
-        _CALLS[key] = ent
+    ent = _entry(x, weight, freqs_cis, eps)
     if ent.contig:
         x = x.clone(memory_format=torch.contiguous_format)
     out = x.new_empty(ent.shape)
@@ -82,6 +73,43 @@ def fused_rms_norm_rope(
     else:
         _lib.check(ent.fn(ctypes.byref(a), torch._C._cuda_getCurrentRawStream(idx)), "qik_rms_rope")
     return out
+
+
+def _rms_rope_qk(query, key, norm_q, norm_k, freqs_cis):
+    """fused_rms_norm_rope of a layer's Q and K (``norm_q`` and ``norm_k`` carry
+    ``weight`` and ``eps``), in one launch when both are of one dtype, head dim
+    and device, else in two."""
+    if query.dtype != key.dtype or query.shape[-1] != key.shape[-1] or query.device != key.device:
+        return (fused_rms_norm_rope(query, norm_q.weight, freqs_cis, norm_q.eps),
+                fused_rms_norm_rope(key, norm_k.weight, freqs_cis, norm_k.eps))
+    args, outs, reads = [], [], []
+    for x, norm in ((query, norm_q), (key, norm_k)):
+        ent = _entry(x, norm.weight, freqs_cis, norm.eps)
+        x = x.clone(memory_format=torch.contiguous_format) if ent.contig else x
+        a = _lib.QikRmsRopeArgs.from_buffer_copy(ent.args)
+        outs.append(x.new_empty(ent.shape))
+        reads.append(x)
+        a.x, a.out = x.data_ptr(), outs[-1].data_ptr()
+        args.append(a)
+    with torch.cuda.device(ent.index):
+        _lib.check(_lib.load().qik_rms_rope_pair(ctypes.byref(args[0]), ctypes.byref(args[1]),
+                                                 torch._C._cuda_getCurrentRawStream(ent.index)), "qik_rms_rope_pair")
+    return outs
+
+
+def _entry(x, weight, freqs_cis, eps) -> _Call:
+    """The prepared call of a (geometry, weight, freqs_cis, eps) key."""
+    key = (x.shape, x.stride(), x.data_ptr() & 15, x.dtype, x.device, eps,
+           weight.data_ptr(), weight._version, weight.dtype, weight.shape, weight.stride(), weight.device,
+           freqs_cis.data_ptr(), freqs_cis._version, freqs_cis.dtype, freqs_cis.shape, freqs_cis.stride(),
+           freqs_cis.device)
+    ent = _CALLS.get(key)
+    if ent is None:
+        ent = _prepare(x, weight, freqs_cis, eps)
+        if len(_CALLS) >= 64:
+            _CALLS.clear()
+        _CALLS[key] = ent
+    return ent
 
 
 class _Call:

@@ -5,7 +5,8 @@ reference processor (qwen_image_kernel/processors.py:39-126), with every device
 step of the attention layer between the projections on this package's HIP
 kernels:
 
-* Q/K: per-head RMSNorm + RoPE, ``fused_rms_norm_rope`` (qik_rms_rope);
+* Q/K: per-head RMSNorm + RoPE (``fused_rms_norm_rope``), both in one launch
+  (qik_rms_rope_pair);
 * prefix extraction: ``layer_cache.store`` (qik_slab_store on a HIP slab);
 * attention: ``block_causal_flash_attention`` (qik_attn_fwd_ws) -- prefill over the
   joint sequence with per-row causal lengths from the segment list, decode of
@@ -22,7 +23,7 @@ from __future__ import annotations
 import torch
 
 from .attention import block_causal_flash_attention, build_prefix_lengths
-from .fused import fused_rms_norm_rope
+from .fused import _rms_rope_qk
 from .kv_cache import _LayerView
 
 __all__ = ["QwenImage21KernelProcessor", "_build_prefix_lengths"]
@@ -71,8 +72,7 @@ class QwenImage21KernelProcessor:
             value = attn.to_v(hidden_states).unflatten(-1, (H, D))
 
         # QK-RMSNorm + RoPE (processors.py:77-79)
-        query = fused_rms_norm_rope(query, attn.norm_q.weight, rotary_emb, attn.norm_q.eps)
-        key = fused_rms_norm_rope(key, attn.norm_k.weight, rotary_emb, attn.norm_k.eps)
+        query, key = _rms_rope_qk(query, key, attn.norm_q, attn.norm_k, rotary_emb)
 
         if kv_cache_mode == "extract" and layer_cache is not None and cache_write_slice is not None:
             k_pre, v_pre = key[:, cache_write_slice], value[:, cache_write_slice]
@@ -101,17 +101,23 @@ class QwenImage21KernelProcessor:
                 else:
                     cache_k, cache_v = layer_cache.get()
                     v_scale = None
-                kv_total = cache_k.shape[1] + key.shape[1]
-                L = torch.full((key.shape[1],), kv_total - 1, dtype=torch.int32, device=query.device)
+                L = self._full_lengths(query, key, cache_k.shape[1], kv_mask)
                 out = block_causal_flash_attention(
                     query, key, value, L, kv_mask, cache_k=cache_k, cache_v=cache_v,
                     cache_v_scale=v_scale, uniform_full=kv_mask is None,
                 )
             else:
                 # no cache: full attention over the whole sequence (:113-122)
-                L = torch.full((key.shape[1],), key.shape[1] - 1, dtype=torch.int32, device=query.device)
+                L = self._full_lengths(query, key, 0, kv_mask)
                 out = block_causal_flash_attention(query, key, value, L, kv_mask, uniform_full=kv_mask is None)
 
         out = out.flatten(2, 3).type_as(query)
         out = attn.to_out[0](out)
         return attn.to_out[1](out)
+
+    @staticmethod
+    def _full_lengths(query, key, prefix: int, kv_mask):
+        """L of rows that see every key; None (no fill launch) where uniform_full says so and L is not read."""
+        if kv_mask is None:
+            return None
+        return torch.full((key.shape[1],), prefix + key.shape[1] - 1, dtype=torch.int32, device=query.device)

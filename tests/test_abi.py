@@ -229,6 +229,21 @@ def test_rms_rope_rejects_before_any_device_call(kw, code):
     assert _lib.load().qik_rms_rope(ctypes.byref(_rope_args(**kw)), None) == code
 
 
+def test_rms_rope_pair_rejects_what_either_call_would():
+    lib = _lib.load()
+    pair = lambda x, y: lib.qik_rms_rope_pair(None if x is None else ctypes.byref(x),  # noqa: E731
+                                              None if y is None else ctypes.byref(y), None)
+    good, empty = _rope_args(), _rope_args(S=0, x=None)
+    assert pair(None, good) == -1 and pair(good, None) == -1
+    for kw in (dict(dtype=7), dict(D=96), dict(x=None), dict(out=8)):
+        bad = _rope_args(**kw)
+        want = lib.qik_rms_rope(ctypes.byref(bad), None)
+        assert want != 0 and pair(bad, good) == want and pair(good, bad) == want
+    assert pair(good, _rope_args(D=64)) == -4                            # one head dim
+    assert pair(good, _rope_args(dtype=_lib.DTYPE_FP16)) == -3           # one dtype
+    assert pair(empty, empty) == 0
+
+
 def test_rms_rope_without_rows_is_a_no_op():
     assert _lib.load().qik_rms_rope(ctypes.byref(_rope_args(S=0, x=None)), None) == 0
 

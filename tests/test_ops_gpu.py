@@ -90,6 +90,32 @@ def test_rms_rope_reads_fused_qkv_views_in_place():
         np.testing.assert_array_equal(_bits(got), _bits(want))
 
 
+@pytest.mark.parametrize("B,S,H,HK,D,dtype", [
+    (1, 1, 1, 1, 128, torch.bfloat16),       # one row each
+    (1, 64, 1, 1, 128, torch.bfloat16),      # whole workgroups of both
+    (2, 67, 3, 5, 64, torch.float16),        # ragged, more K rows than Q rows
+    (1, 33, 7, 2, 256, torch.bfloat16),      # fewer
+    (1, 130, 4, 4, 32, torch.bfloat16),
+])
+@pytest.mark.parametrize("strided", [False, True])
+def test_rms_rope_pair_equals_two_calls(B, S, H, HK, D, dtype, strided):
+    """Q and K in one launch give the bits of two calls, read in place or not."""
+    from types import SimpleNamespace
+
+    from qwen_image_kernel_amd.fused import _rms_rope_qk
+    _flush(f"case rms_rope pair {B}x{S}x{H},{HK}x{D} {dtype} strided={strided}")
+    g = torch.Generator().manual_seed(21 + S)
+    both = torch.randn(B, S, H + HK, D, generator=g).to(dtype).to(DEV)
+    q, k = both[:, :, :H], both[:, :, H:]
+    if not strided:
+        q, k = q.contiguous(), k.contiguous()
+    nq, nk = (SimpleNamespace(weight=(torch.randn(D, generator=g) * 0.3 + 1).to(DEV), eps=e) for e in (1e-6, 1e-5))
+    freqs = orr.rope_freqs(S, D).to(DEV)
+    gq, gk = _rms_rope_qk(q, k, nq, nk, freqs)
+    np.testing.assert_array_equal(_bits(gq), _bits(qik.fused_rms_norm_rope(q, nq.weight, freqs, 1e-6)))
+    np.testing.assert_array_equal(_bits(gk), _bits(qik.fused_rms_norm_rope(k, nk.weight, freqs, 1e-5)))
+
+
 def test_rms_rope_rejects_bad_freqs():
     x = torch.zeros(1, 8, 2, 128, dtype=torch.bfloat16, device=DEV)
     with pytest.raises(ValueError):
