@@ -239,28 +239,72 @@ struct CopyParams {
   int64_t* len_dst;  // NULL, or where the first launch writes P
 };
 
-// One 16-byte chunk g of the copy of tensor `which` (0 = K, 1 = V).
-__device__ __forceinline__ void copy_chunk(const CopyParams& p, const int which, const int64_t g) {
-  const int tpr = p.row_bytes / 16;
-  const int64_t row = g / tpr;
-  const int t = (int)(g % tpr);
+// CR passes of THREADS / (row_bytes / 16) rows per workgroup, their loads issued
+// before any store; (b, h, p) of the first row by division, then stepped.  The
+// slab is read again only by later decode steps, layers and megabytes away: its
+// rows are stored non-temporally and leave the caches to what is read next.
+// Bound by the copy rate: an fp8 store of 2 x 3328 x 24 x 128 (220 MB with the
+// V reads) 40.4 us with plain stores, 30.0 with these; 1 x 2560 15.5 / 14.3.
+template <int THREADS, int CR>
+__device__ __forceinline__ void copy_rows(const CopyParams& p, const int which, const int64_t block) {
+  const int tpr = p.row_bytes / 16;   // 4 .. 32 threads per row
+  const int rps = THREADS / tpr;
+  const int t = (int)threadIdx.x % tpr;
+  const int64_t row = block * (rps * CR) + (int)threadIdx.x / tpr;
   if (row >= p.rows) return;
-  const int64_t pp = row % p.P;  // destination row order: b, h, p
-  const int64_t bh = row / p.P;
-  const int64_t h = bh % p.H;
-  const int64_t b = bh / p.H;
-  const u32x4 v = *reinterpret_cast<const u32x4*>(
-      p.src[which] + (b * p.ss[which][0] + pp * p.ss[which][1] + h * p.ss[which][2]) * 2 + t * 16);
-  *reinterpret_cast<u32x4*>(p.dst[which] + (b * p.sd[which][0] + h * p.sd[which][1] + pp * p.sd[which][2]) * 2 +
-                            t * 16) = v;
+  int64_t pp, h, b;  // destination row order: b, h, p
+  if (p.rows <= (int64_t)UINT_MAX) {
+    const unsigned bh = (unsigned)row / (unsigned)p.P;
+    pp = (unsigned)row - bh * (unsigned)p.P;
+    b = bh / (unsigned)p.H;
+    h = bh - (unsigned)b * (unsigned)p.H;
+  } else {
+    const int64_t bh = row / p.P;
+    pp = row - bh * p.P;
+    b = bh / p.H;
+    h = bh - b * p.H;
+  }
+  const int64_t* const ss = p.ss[which];
+  const int64_t* const sd = p.sd[which];
+  int64_t so = b * ss[0] + pp * ss[1] + h * ss[2];
+  int64_t dofs = b * sd[0] + h * sd[1] + pp * sd[2];
+  u32x4 v[CR];
+  int64_t at[CR];
+  bool live[CR];
+#pragma unroll
+  for (int u = 0; u < CR; ++u) {
+    live[u] = row + u * rps < p.rows;
+    at[u] = dofs;
+    v[u] = u32x4{0u, 0u, 0u, 0u};
+    if (live[u]) v[u] = *reinterpret_cast<const u32x4*>(p.src[which] + so * 2 + t * 16);
+    if (u + 1 < CR) {
+      pp += rps;
+      so += rps * ss[1];
+      dofs += rps * sd[2];
+      while (pp >= p.P) {
+        pp -= p.P;
+        so += ss[2] - p.P * ss[1];
+        dofs += sd[1] - p.P * sd[2];
+        if (++h == p.H) {
+          h = 0;
+          so += ss[0] - p.H * ss[2];
+          dofs += sd[0] - p.H * sd[1];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < CR; ++u)
+    if (live[u]) __builtin_nontemporal_store(v[u], reinterpret_cast<u32x4*>(p.dst[which] + at[u] * 2 + t * 16));
 }
 
+template <int CR>
 __global__ void __launch_bounds__(NTHREADS) slab_copy_kernel(const CopyParams p) {
   const int which = blockIdx.y;
   const int64_t g = (int64_t)blockIdx.x * NTHREADS + threadIdx.x;
   if (p.zero != nullptr && which == 0 && g < p.nzero) p.zero[g] = 0.0f;
   if (p.len_dst != nullptr && which == 0 && g == 0) *p.len_dst = p.P;
-  copy_chunk(p, which, g);
+  copy_rows<NTHREADS, CR>(p, which, blockIdx.x);
 }
 
 // fp8 V over `chunks` workgroups per (b, h), workgroup c owning rows
@@ -271,9 +315,11 @@ __global__ void __launch_bounds__(NTHREADS) slab_copy_kernel(const CopyParams p)
 //   qik_slab_store: slab_scale_fp8_kernel maxes each chunk's scale atomically
 //     into scale[b*H + h] (zeroed by the copy launch before), then
 //     slab_quant_fp8_kernel writes the codes (three launches with the copy);
-//   qik_slab_store_ws: slab_copy_scale_kernel copies K and writes each chunk's
-//     scale into the workspace, then slab_quant_fp8_kernel takes the largest of
-//     its head's and writes the codes and the scale (two launches).
+//   qik_slab_store_ws: each chunk's scale goes into the workspace, then the
+//     codes' blocks take the largest of their head's and one of them writes it
+//     (two launches).  K is copied beside the scales when V is small
+//     (slab_copy_scale_kernel, slab_quant_fp8_kernel), beside the codes when it
+//     is large (slab_partial_scale_kernel, slab_quant_copy_kernel).
 struct QuantParams {
   const char* v;     // bf16 or fp16 [B, P, H, D]
   char* dst;         // fp8 slab V of the layer
@@ -351,16 +397,17 @@ __global__ void __launch_bounds__(QTHREADS) slab_scale_fp8_kernel(const QuantPar
   if (threadIdx.x == 0) atomicMax(reinterpret_cast<unsigned*>(p.scale) + blockIdx.x / p.chunks, __float_as_uint(sc));
 }
 
-// Workspace form, first launch: blocks [0, ncopy) copy K (QTHREADS 16-byte
+constexpr int STORE_CR = 4;
+
+// Small V, first launch: blocks [0, ncopy) copy K (STORE_CR * QTHREADS 16-byte
 // chunks each), the others write their chunk's scale into p.partial.  Every
 // partial is written, so the workspace needs no clearing.
 template <int D, bool FP16>
 __global__ void __launch_bounds__(QTHREADS) slab_copy_scale_kernel(const CopyParams cp, const QuantParams p,
                                                                    const int ncopy) {
   if ((int)blockIdx.x < ncopy) {
-    const int64_t g = (int64_t)blockIdx.x * QTHREADS + threadIdx.x;
-    if (cp.len_dst != nullptr && g == 0) *cp.len_dst = cp.P;
-    copy_chunk(cp, 0, g);
+    if (cp.len_dst != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *cp.len_dst = cp.P;
+    copy_rows<QTHREADS, STORE_CR>(cp, 0, blockIdx.x);
     return;
   }
   const int bx = (int)blockIdx.x - ncopy;
@@ -368,8 +415,16 @@ __global__ void __launch_bounds__(QTHREADS) slab_copy_scale_kernel(const CopyPar
   if (threadIdx.x == 0) p.partial[bx] = sc;
 }
 
+// Large V, first launch: the chunks' scales alone.
 template <int D, bool FP16>
-__global__ void __launch_bounds__(QTHREADS) slab_quant_fp8_kernel(const QuantParams p) {
+__global__ void __launch_bounds__(QTHREADS) slab_partial_scale_kernel(const QuantParams p) {
+  const float sc = chunk_scale<D, FP16>(p, blockIdx.x);
+  if (threadIdx.x == 0) p.partial[blockIdx.x] = sc;
+}
+
+// The codes of chunk c of head bh.
+template <int D, bool FP16>
+__device__ __forceinline__ void quant_chunk(const QuantParams& p) {
 #pragma clang fp contract(off)
   constexpr int TPR = D / 8;             // threads per row
   constexpr int RPS = QTHREADS / TPR;    // rows per step
@@ -444,12 +499,31 @@ __global__ void __launch_bounds__(QTHREADS) slab_quant_fp8_kernel(const QuantPar
       lo = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], lo, true);
       int hi = __builtin_amdgcn_cvt_pk_fp8_f32(q[4], q[5], 0, false);
       hi = __builtin_amdgcn_cvt_pk_fp8_f32(q[6], q[7], hi, true);
-      *reinterpret_cast<u32x2*>(dst + (q0 + u * RPS) * p.sd[2]) = u32x2{(unsigned)lo, (unsigned)hi};
+      __builtin_nontemporal_store(u32x2{(unsigned)lo, (unsigned)hi},
+                                  reinterpret_cast<u32x2*>(dst + (q0 + u * RPS) * p.sd[2]));
     }
     q0 += U * RPS;
     if (q0 >= p1) break;
     load_batch(q0);
   }
+}
+
+template <int D, bool FP16>
+__global__ void __launch_bounds__(QTHREADS) slab_quant_fp8_kernel(const QuantParams p) {
+  quant_chunk<D, FP16>(p);
+}
+
+// Large V, second launch: blocks [0, nquant) write the codes, the others copy K.
+template <int D, bool FP16>
+__global__ void __launch_bounds__(QTHREADS) slab_quant_copy_kernel(const CopyParams cp, const QuantParams p,
+                                                                   const int nquant) {
+  if ((int)blockIdx.x < nquant) {
+    quant_chunk<D, FP16>(p);
+    return;
+  }
+  const int block = (int)blockIdx.x - nquant;
+  if (cp.len_dst != nullptr && block == 0 && threadIdx.x == 0) *cp.len_dst = cp.P;
+  copy_rows<QTHREADS, STORE_CR>(cp, 0, block);
 }
 
 // CUs of the current device (0 if the runtime cannot say), cached per device
@@ -618,8 +692,12 @@ int store(const qik_slab_store_args* a, float* partial, hipStream_t s) {
   cp.zero = (fp8 && partial == nullptr) ? a->v_scale : nullptr;
   cp.nzero = a->B * a->H;
   const int64_t threads = rows * (a->D * 2 / 16);
-  const int64_t grid = (threads + NTHREADS - 1) / NTHREADS;
-  if (grid > (int64_t)UINT_MAX) return QIK_ERR_SHAPE;
+  // four rows per copy thread where that leaves two workgroups per CU (2560 x 24
+  // x 128 10.97 us against 11.44 with one), else one (2 x 700 x 12 x 64 3.2 / 3.7)
+  const int64_t per1 = (threads + NTHREADS - 1) / NTHREADS;
+  const bool four = per1 >= 8 * (int64_t)std::max(device_cus(), 1);
+  const int64_t grid = four ? (per1 + 3) / 4 : per1;
+  if (per1 > (int64_t)UINT_MAX) return QIK_ERR_SHAPE;
 
   QuantParams qp;
   memset(&qp, 0, sizeof(qp));
@@ -652,30 +730,48 @@ int store(const qik_slab_store_args* a, float* partial, hipStream_t s) {
   const void* fq = quant_fns[kix];
 
   if (fp8 && partial != nullptr) {
-    // K copy and the chunks' scales in one launch, then the codes.  The copy
-    // blocks are rounded up to a multiple of 8 (the extra ones find no row and
-    // return), so chunk c runs on XCD c % 8 in both launches (the dispatcher
-    // deals block b to XCD b % 8): the codes launch re-reads its V rows from
-    // the L2 that the scale launch read them through.
-    const int64_t ncopy = ((threads + QTHREADS - 1) / QTHREADS + 7) / 8 * 8;
-    if (ncopy + heads * chunks > (int64_t)INT_MAX) return QIK_ERR_SHAPE;
-    int nc = (int)ncopy;
-    void* args2[] = {&cp, &qp, &nc};
+    // Chunk c runs on XCD c % 8 in both launches (the dispatcher deals block b
+    // to XCD b % 8; the copy's blocks are rounded up to a multiple of 8, the
+    // extra ones find no row), so the codes launch re-reads its V rows from the
+    // L2 that the scale launch read them through.  K goes with the codes from
+    // LARGE_V bytes of V on: the codes' blocks alone are too short a launch to
+    // fill the memory's time there (V of 15.7 MB 14.3 us against 15.7 with K
+    // beside the scales, 51 MB 30.0 / 32.7; below, the scales alone are the
+    // short launch: 4.3 MB 10.3 / 9.2, 4.6 MB 10.3 / 9.3).
+    constexpr int64_t LARGE_V = 8 << 20;
+    const bool large = threads * 16 >= LARGE_V;
+    const int64_t ncopy = ((threads + QTHREADS * STORE_CR - 1) / (QTHREADS * STORE_CR) + 7) / 8 * 8;
+    const int64_t nquant = heads * chunks;
+    if (ncopy + nquant > (int64_t)INT_MAX) return QIK_ERR_SHAPE;
+    int own = (int)(large ? nquant : ncopy);  // blocks of the two-part launch's first part
+    void* both[] = {&cp, &qp, &own};
     const void* const copy_scale_fns[8] = {
         (const void*)slab_copy_scale_kernel<32, false>,  (const void*)slab_copy_scale_kernel<32, true>,
         (const void*)slab_copy_scale_kernel<64, false>,  (const void*)slab_copy_scale_kernel<64, true>,
         (const void*)slab_copy_scale_kernel<128, false>, (const void*)slab_copy_scale_kernel<128, true>,
         (const void*)slab_copy_scale_kernel<256, false>, (const void*)slab_copy_scale_kernel<256, true>};
-    const void* fc = copy_scale_fns[kix];
-    if (hipLaunchKernel(fc, dim3((unsigned)(ncopy + heads * chunks)), dim3(QTHREADS), args2, 0, s) != hipSuccess)
-      return QIK_ERR_LAUNCH;
-    return hipLaunchKernel(fq, dim3((unsigned)(heads * chunks)), dim3(QTHREADS), qargs, 0, s) == hipSuccess
-               ? QIK_OK : QIK_ERR_LAUNCH;
+    const void* const partial_fns[8] = {
+        (const void*)slab_partial_scale_kernel<32, false>,  (const void*)slab_partial_scale_kernel<32, true>,
+        (const void*)slab_partial_scale_kernel<64, false>,  (const void*)slab_partial_scale_kernel<64, true>,
+        (const void*)slab_partial_scale_kernel<128, false>, (const void*)slab_partial_scale_kernel<128, true>,
+        (const void*)slab_partial_scale_kernel<256, false>, (const void*)slab_partial_scale_kernel<256, true>};
+    const void* const quant_copy_fns[8] = {
+        (const void*)slab_quant_copy_kernel<32, false>,  (const void*)slab_quant_copy_kernel<32, true>,
+        (const void*)slab_quant_copy_kernel<64, false>,  (const void*)slab_quant_copy_kernel<64, true>,
+        (const void*)slab_quant_copy_kernel<128, false>, (const void*)slab_quant_copy_kernel<128, true>,
+        (const void*)slab_quant_copy_kernel<256, false>, (const void*)slab_quant_copy_kernel<256, true>};
+    const dim3 part((unsigned)nquant), whole((unsigned)(ncopy + nquant)), block(QTHREADS);
+    const hipError_t e1 = large ? hipLaunchKernel(partial_fns[kix], part, block, qargs, 0, s)
+                                : hipLaunchKernel(copy_scale_fns[kix], whole, block, both, 0, s);
+    if (e1 != hipSuccess) return QIK_ERR_LAUNCH;
+    const hipError_t e2 = large ? hipLaunchKernel(quant_copy_fns[kix], whole, block, both, 0, s)
+                                : hipLaunchKernel(fq, part, block, qargs, 0, s);
+    return e2 == hipSuccess ? QIK_OK : QIK_ERR_LAUNCH;
   }
 
   void* cargs[] = {&cp};
-  hipError_t e = hipLaunchKernel(reinterpret_cast<const void*>(slab_copy_kernel), dim3((unsigned)grid, fp8 ? 1 : 2),
-                                 dim3(NTHREADS), cargs, 0, s);
+  const void* const copy_fn = four ? (const void*)slab_copy_kernel<4> : (const void*)slab_copy_kernel<1>;
+  hipError_t e = hipLaunchKernel(copy_fn, dim3((unsigned)grid, fp8 ? 1 : 2), dim3(NTHREADS), cargs, 0, s);
   if (e != hipSuccess) return QIK_ERR_LAUNCH;
   if (!fp8) return QIK_OK;
   const void* const scale_fns[8] = {

@@ -116,6 +116,64 @@ def test_rms_rope_pair_equals_two_calls(B, S, H, HK, D, dtype, strided):
     np.testing.assert_array_equal(_bits(gk), _bits(qik.fused_rms_norm_rope(k, nk.weight, freqs, 1e-5)))
 
 
+@pytest.mark.parametrize("P", [1, 7, 31, 32, 33, 64, 127, 128, 129, 255])
+@pytest.mark.parametrize("D,v_fp8", [(32, False), (64, True), (128, True), (128, False), (256, True)])
+def test_slab_store_row_steps(P, D, v_fp8):
+    """Prefix lengths around a copy thread's row step (8 to 128 rows) and a workgroup's
+    share, so that the step wraps over positions, heads and batches; a slab with
+    rows past the prefix, which keep what they held."""
+    _flush(f"case slab store rows P={P} D={D} fp8={v_fp8}")
+    B, H = 2, 3
+    g = torch.Generator().manual_seed(31 + P + D)
+    k, v = (torch.randn(B, P, 3 * H, D, generator=g).to(torch.bfloat16).to(DEV)[:, :, H:2 * H] for _ in range(2))
+    cache = qik.ContiguousKVCache(1, B, P + 16, H, D, v_fp8=v_fp8, device=DEV)
+    layer = cache.get_layer(0)
+    layer.store(torch.full((B, P + 16, H, D), 3.0, dtype=torch.bfloat16, device=DEV),
+                torch.full((B, P + 16, H, D), 2.0, dtype=torch.bfloat16, device=DEV))
+    full_k, full_v, _ = layer.views()
+    layer.store(k, v)
+    kc, vc, sc = layer.views()
+    assert torch.equal(kc, k) and (full_k[:, P:] == 3.0).all()
+    if not v_fp8:
+        assert torch.equal(vc, v) and (full_v[:, P:] == 2.0).all()
+        return
+    codes, scale = of.quantize_per_head(v.float().cpu().numpy())
+    np.testing.assert_array_equal(sc.cpu().numpy(), scale)
+    np.testing.assert_array_equal(vc.transpose(1, 2).contiguous().view(torch.uint8).cpu().numpy(), codes)
+
+
+@pytest.mark.parametrize("B,P,H,D,v_fp8", [
+    (1, 1365, 24, 128, True),   # V just below 8 MiB: K copied beside the scales
+    (1, 1366, 24, 128, True),   # just above: beside the codes
+    (2, 1400, 12, 128, True),
+    (1, 2730, 24, 64, True),
+    (1, 2731, 24, 64, True),
+    (1, 5462, 24, 128, False),  # four rows per copy thread
+    (1, 5461, 3, 32, False),    # one
+])
+def test_slab_store_launch_forms(B, P, H, D, v_fp8):
+    """Both sides of each line between the store's launch forms, through the workspace
+    entry point and the one without."""
+    _flush(f"case slab store forms {B}x{P}x{H}x{D} fp8={v_fp8}")
+    g = torch.Generator(device=DEV).manual_seed(41 + P)
+    k, v = (torch.randn(B, P, H, D, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    caches = [qik.ContiguousKVCache(1, B, P + 8, H, D, v_fp8=v_fp8, device=DEV) for _ in range(2)]
+    caches[0].get_layer(0).store(k, v)
+    a, _keep = caches[1].get_layer(0).store_args(k, v, P)
+    _lib.check(_lib.load().qik_slab_store(ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)),
+               "qik_slab_store")
+    torch.cuda.synchronize()
+    for c in caches:
+        assert torch.equal(c.k_buf[0][:, :, :P], k.transpose(1, 2))
+        if v_fp8:
+            scale = (v.float().abs().amax(dim=(1, 3)) * torch.tensor(1.0 / 448.0, device=DEV)).clamp_min(1e-12)
+            assert torch.equal(c.v_scale[0].reshape(B, H), scale)
+            want = (v.float() / scale[:, None, :, None]).clamp(-448.0, 448.0).to(torch.float8_e4m3fn)
+            assert torch.equal(c.v_buf[0].view(torch.uint8)[:, :, :P], want.transpose(1, 2).view(torch.uint8))
+        else:
+            assert torch.equal(c.v_buf[0][:, :, :P], v.transpose(1, 2))
+
+
 def test_rms_rope_rejects_bad_freqs():
     x = torch.zeros(1, 8, 2, 128, dtype=torch.bfloat16, device=DEV)
     with pytest.raises(ValueError):
