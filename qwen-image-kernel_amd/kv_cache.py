@@ -158,18 +158,22 @@ class _LayerView:
 
     def get(self):
         """(k, v) as [B, P, H, D] strided views."""
-        P = self._c._host_lengths[self._layer]
-        k = self._c.k_buf[self._layer, :, :, :P, :].transpose(1, 2)
-        v = self._c.v_buf[self._layer, :, :, :P, :].transpose(1, 2)
-        return k, v
+        c = self._c
+        P = c._host_lengths[self._layer]
+        return self._prefix(c.k_buf, P), self._prefix(c.v_buf, P)
+
+    def _prefix(self, buf: torch.Tensor, P: int) -> torch.Tensor:
+        """``buf[layer, :, :, :P, :].transpose(1, 2)`` in one view op (1.7 us of host time for
+        the chain's 5.6, of which a store and its views have two)."""
+        sl, sb, sh, sp, sd = buf.stride()
+        _, B, H, cap, D = buf.shape
+        return buf.as_strided((B, P if P < cap else cap, H, D), (sb, sp, sh, sd),
+                              buf.storage_offset() + self._layer * sl)
 
     def views(self):
         """(k, v, v_scale_or_None) for block_causal_flash_attention."""
-        P = self._c._host_lengths[self._layer]
-        k = self._c.k_buf[self._layer, :, :, :P, :].transpose(1, 2)
-        v = self._c.v_buf[self._layer, :, :, :P, :].transpose(1, 2)
-        scale = self._c.v_scale[self._layer] if self._c.v_fp8 else None
-        return k, v, scale
+        k, v = self.get()
+        return k, v, (self._c.v_scale[self._layer] if self._c.v_fp8 else None)
 
 
 class ContiguousKVCache:

@@ -506,6 +506,24 @@ def test_slab_store_fp8_takes_fp16_and_cache_rejects_other_dtypes():
             qik.ContiguousKVCache(1, 1, 16, 2, 128, device="cuda", dtype=dt)
 
 
+@pytest.mark.parametrize("P", [0, 1, 23, 32])
+def test_slab_views_are_the_indexed_views(P):
+    """views() and get() give the same views of the slab as indexing it: shape, strides,
+    address and writes through them."""
+    import torch
+    import qwen_image_kernel_amd as qik
+    g = torch.Generator().manual_seed(7)
+    cache = qik.ContiguousKVCache(3, 2, 32, 4, 64, v_fp8=False, device="cpu")
+    layer = cache.get_layer(1)
+    layer.store(*(torch.randn(2, P, 4, 64, generator=g).to(torch.bfloat16) for _ in range(2)))
+    for k, v in (layer.get(), layer.views()[:2]):
+        for got, buf in ((k, cache.k_buf), (v, cache.v_buf)):
+            want = buf[1, :, :, :P, :].transpose(1, 2)
+            assert got.shape == want.shape and got.stride() == want.stride() and got.dtype == want.dtype
+            assert got.storage_offset() == want.storage_offset() and torch.equal(got, want)
+            assert got.untyped_storage().data_ptr() == buf.untyped_storage().data_ptr()
+
+
 @pytest.mark.parametrize("v_fp8", [False, True])
 def test_cpu_slab_takes_any_float_dtype_like_the_reference(v_fp8):
     """A CPU slab is stored by the reference's torch ops (kv_cache.py:30-45),
