@@ -361,7 +361,11 @@ __device__ __forceinline__ Params reread_args() {
 // launch for row blocks that fit the CUs once; no workspace, no queue).
 // D = 256 holds 128 accumulator registers per lane and runs one workgroup per
 // CU (one wave per SIMD); the other head dims run two.
-template <int D, bool FP16, bool V_FP8, bool KV, int KSPLIT>
+// MANY: items of more than two pieces (a kernel of its own, KSPLIT = 1 and D <=
+// 128 only: the merge of many pieces changes the register allocation of the
+// kernel it is in; 264 fp16 row blocks with a key mask ran 1.5% slower in one
+// kernel for both).
+template <int D, bool FP16, bool V_FP8, bool KV, int KSPLIT, bool MANY>
 __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ? 2 : 1)
     attn_fwd_kernel(const Params args) {
   constexpr int CH = D / 8;              // 16-byte chunks per row (8 elements)
@@ -382,9 +386,7 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
   static_assert(BN == 64, "one key_valid byte per lane of wave 0");
 
   static_assert(KSPLIT == 1 || KSPLIT == 2, "one or two groups of waves");
-  // items of more than two pieces: not in the two-group kernel, and not at
-  // D = 256 (max_pieces), whose registers are full
-  constexpr bool MANY = KSPLIT == 1 && D <= 128;
+  static_assert(!MANY || (KSPLIT == 1 && D <= 128), "many pieces: one group, and registers to merge them in");
   // per group: K stage 0, K stage 1, V stage 0, V stage 1 (one contiguous block)
   __shared__ u32x4 stg[4 * KSPLIT][TILE_BYTES / 16];
   __shared__ uint32_t skv[KSPLIT][2][BN / 4];   // key_valid bytes of each stage's tile (4 per word)
@@ -590,8 +592,8 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
       // pieces (T, and so the split, is the same for both pieces of the item)
       bool split = wk.group >= 0 && T >= (KSPLIT == 1 ? SPLIT_MIN_TILES : PIECE_MIN_TILES);
       if constexpr (KSPLIT == 1) {
-        const int ns = p.plan.ns;
-        if (MANY && ns > 2) {
+        [[maybe_unused]] const int ns = p.plan.ns;
+        if (MANY) {
           split = split && T >= MANY_MIN_TILES * ns;
           g0 = split ? T * wk.piece / ns : 0;
           g1 = split ? T * (wk.piece + 1) / ns : T;
@@ -946,12 +948,14 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
       // the other piece's state; the two combine in piece order, the same
       // arithmetic whichever of them arrived last (in the two-group kernel
       // group 0 holds the workgroup's state and stores the rows)
-      if (MANY && pe.plan.ns > 2) {
+      if constexpr (MANY) {
         // ns pieces: every (m, l) first, then the accumulators piece by piece,
         // this piece's own in its turn.  Explicit fmas: the compiler takes the
         // products of its own state out of the loop otherwise, and rounds them
         // where a loaded piece's are fused, so that the bits would depend on
-        // which piece merges.
+        // which piece merges.  Half of the accumulators per pass: with all of
+        // them the merge needs three sets of 64 registers and the kernel spills
+        // 16 to 30 (2 x 24 heads x 2772 rows 359.3 us, 355.2 with halves).
         const int ns = pe.plan.ns;
         float mm = m_run;
         for (int pc = 0; pc < ns; ++pc) {
@@ -961,36 +965,41 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
                                                        sl, (uint32_t)(OB + tid * 8), 0, SC1))[0]);
         }
         l_part = 0.0f;
-        f32x16 macc[DBLK];
+        constexpr int DH = (DBLK + 1) / 2;  // blocks per pass
 #pragma unroll
-        for (int db = 0; db < DBLK; ++db) macc[db] = f32x16{};
-        for (int pc = 0; pc < ns; ++pc) {
-          if (pc == wk.piece) {
-            const float a = (m_run == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(m_run - mm);
-            l_part = __builtin_fmaf(l_run, a, l_part);
+        for (int d0 = 0; d0 < DBLK; d0 += DH) {
+          f32x16 macc[DH];
 #pragma unroll
-            for (int db = 0; db < DBLK; ++db)
+          for (int db = 0; db < DH; ++db) macc[db] = f32x16{};
+          for (int pc = 0; pc < ns; ++pc) {
+            if (pc == wk.piece) {
+              const float a = (m_run == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(m_run - mm);
+              if (d0 == 0) l_part = __builtin_fmaf(l_run, a, l_part);
 #pragma unroll
-              for (int i = 0; i < 16; ++i) macc[db][i] = __builtin_fmaf(oacc[db][i], a, macc[db][i]);
-            continue;
+              for (int db = 0; db < DH; ++db)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) macc[db][i] = __builtin_fmaf(oacc[d0 + db][i], a, macc[db][i]);
+              continue;
+            }
+            const auto sl = make_rsrc(gslots + pc * SB, SB);
+            const f32x2 ml = __builtin_bit_cast(
+                f32x2, __builtin_amdgcn_raw_buffer_load_b64(sl, (uint32_t)(OB + tid * 8), 0, SC1));
+            f32x4 v[DH * 4];
+#pragma unroll
+            for (int i = 0; i < DH * 4; ++i)
+              v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                   sl, (uint32_t)(((d0 * 4 + i) * NTHREADS + tid) * 16), 0, SC1));
+            const float a = (ml[0] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(ml[0] - mm);
+            if (d0 == 0) l_part = __builtin_fmaf(ml[1], a, l_part);
+#pragma unroll
+            for (int i = 0; i < DH * 4; ++i)
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                macc[i / 4][4 * (i % 4) + e] = __builtin_fmaf(v[i][e], a, macc[i / 4][4 * (i % 4) + e]);
           }
-          const auto sl = make_rsrc(gslots + pc * SB, SB);
-          const f32x2 ml = __builtin_bit_cast(
-              f32x2, __builtin_amdgcn_raw_buffer_load_b64(sl, (uint32_t)(OB + tid * 8), 0, SC1));
-          f32x4 v[DBLK * 4];
 #pragma unroll
-          for (int i = 0; i < DBLK * 4; ++i)
-            v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                 sl, (uint32_t)((i * NTHREADS + tid) * 16), 0, SC1));
-          const float a = (ml[0] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(ml[0] - mm);
-          l_part = __builtin_fmaf(ml[1], a, l_part);
-#pragma unroll
-          for (int i = 0; i < DBLK * 4; ++i)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) macc[i / 4][4 * (i % 4) + e] = __builtin_fmaf(v[i][e], a, macc[i / 4][4 * (i % 4) + e]);
+          for (int db = 0; db < DH; ++db) oacc[d0 + db] = macc[db];
         }
-#pragma unroll
-        for (int db = 0; db < DBLK; ++db) oacc[db] = macc[db];
       } else if (KSPLIT == 1 || grp == 0) {
         const auto other = make_rsrc(gslots + (wk.piece ^ 1) * SB, SB);
         const f32x2 mlo = __builtin_bit_cast(
@@ -1137,33 +1146,40 @@ __global__ void zero16_kernel(u32x4* p, int n16) {
 
 typedef void (*kernel_fn)(Params);
 
-template <int D, bool KV, int KS>
+// How a launch runs its row blocks: one unit per workgroup or a queue of units
+// (ONE), the queue with items of more than two pieces (PIECES), or a two-group
+// workgroup per row block (GROUPS).  At D = 256 ONE only: two groups' LDS
+// stages are more than a CU holds, and its registers leave no room to merge
+// many pieces.
+enum class Form { ONE, PIECES, GROUPS };
+
+template <int D, bool KV, int KS, bool MANY>
 kernel_fn pick_kernel(bool fp16, bool vfp8) {
-  if (fp16) return attn_fwd_kernel<D, true, false, KV, KS>;
-  if (vfp8) return attn_fwd_kernel<D, false, true, KV, KS>;
-  return attn_fwd_kernel<D, false, false, KV, KS>;
+  if (fp16) return attn_fwd_kernel<D, true, false, KV, KS, MANY>;
+  if (vfp8) return attn_fwd_kernel<D, false, true, KV, KS, MANY>;
+  return attn_fwd_kernel<D, false, false, KV, KS, MANY>;
 }
 
 // key_valid is a template parameter: without a mask the kernel carries none
 // of its code (the tile loop is then the same as with no mask support at all)
 template <int D>
-kernel_fn pick_kernel(bool fp16, bool vfp8, bool kv, bool two_groups) {
+kernel_fn pick_kernel(bool fp16, bool vfp8, bool kv, Form form) {
   if constexpr (D <= 128) {
-    if (two_groups) return kv ? pick_kernel<D, true, 2>(fp16, vfp8) : pick_kernel<D, false, 2>(fp16, vfp8);
+    if (form == Form::GROUPS) return kv ? pick_kernel<D, true, 2, false>(fp16, vfp8) : pick_kernel<D, false, 2, false>(fp16, vfp8);
+    if (form == Form::PIECES) return kv ? pick_kernel<D, true, 1, true>(fp16, vfp8) : pick_kernel<D, false, 1, true>(fp16, vfp8);
   }
-  return kv ? pick_kernel<D, true, 1>(fp16, vfp8) : pick_kernel<D, false, 1>(fp16, vfp8);
+  return kv ? pick_kernel<D, true, 1, false>(fp16, vfp8) : pick_kernel<D, false, 1, false>(fp16, vfp8);
 }
 
-// The two-group form needs two groups' LDS stages in one workgroup (256 KiB
-// at D = 256, more than a CU holds): not at D = 256.
 inline bool two_group_dim(int64_t D) { return D <= 128; }
+inline int max_pieces_dim(int64_t D) { return D <= 128 ? MAX_PIECES : 2; }
 
-kernel_fn pick_kernel_d(int64_t D, bool fp16, bool vfp8, bool kv, bool two_groups) {
+kernel_fn pick_kernel_d(int64_t D, bool fp16, bool vfp8, bool kv, Form form) {
   switch (D) {
-    case 32: return pick_kernel<32>(fp16, vfp8, kv, two_groups);
-    case 64: return pick_kernel<64>(fp16, vfp8, kv, two_groups);
-    case 128: return pick_kernel<128>(fp16, vfp8, kv, two_groups);
-    default: return pick_kernel<256>(fp16, vfp8, kv, false);
+    case 32: return pick_kernel<32>(fp16, vfp8, kv, form);
+    case 64: return pick_kernel<64>(fp16, vfp8, kv, form);
+    case 128: return pick_kernel<128>(fp16, vfp8, kv, form);
+    default: return pick_kernel<256>(fp16, vfp8, kv, Form::ONE);
   }
 }
 
@@ -1282,7 +1298,7 @@ int plan_launch(const qik_attn_args* a, bool split, Launch* L) {
   const bool fp16 = a->dtype == QIK_DTYPE_FP16;
   const bool vfp8 = (a->flags & QIK_V_CACHE_FP8) != 0;
   const bool kv = (a->flags & QIK_HAS_KEY_VALID) != 0;
-  L->fn = pick_kernel_d(a->D, fp16, vfp8, kv, false);
+  L->fn = pick_kernel_d(a->D, fp16, vfp8, kv, Form::ONE);
   L->slot = slot_bytes_d(a->D);
   L->ws_bytes = 0;
   L->ctl_bytes = 0;
@@ -1296,7 +1312,7 @@ int plan_launch(const qik_attn_args* a, bool split, Launch* L) {
   if (split && two_group_dim(a->D) && n <= cus) {
     // row blocks fit the CUs once: one two-group workgroup per row block, its
     // KV tiles split between the groups and merged in LDS (no workspace) ...
-    L->fn = pick_kernel_d(a->D, fp16, vfp8, kv, true);
+    L->fn = pick_kernel_d(a->D, fp16, vfp8, kv, Form::GROUPS);
     L->threads = 2 * NTHREADS;
     if (2 * n <= cus && cus >= nx) {
       // ... or, with at most half the CUs' worth of row blocks (one GPU's share
@@ -1318,12 +1334,14 @@ int plan_launch(const qik_attn_args* a, bool split, Launch* L) {
   if (split) {
     const int st = slots_per_xcd(L->fn, pick_index((int)a->D, fp16, vfp8, kv), &sx);
     if (st != QIK_OK) return st;
-    L->plan = make_plan((int)n, (int)nmb, sx, 1, (a->flags & QIK_UNIFORM_L) ? 0 : 1, nx, a->D <= 128 ? MAX_PIECES : 2);
+    L->plan = make_plan((int)n, (int)nmb, sx, 1, (a->flags & QIK_UNIFORM_L) ? 0 : 1, nx,
+                        max_pieces_dim(a->D));
     // queue positions are mapped through loc * nx + x, which must fit an
     // int, and the arrival words must fit the fixed control region (the same
     // for every shape, so that no launch leaves slot data where another
     // launch keeps its control words)
     if ((int64_t)nx * L->plan.wpx <= INT_MAX && 2 * NXCD_MAX + L->plan.ngroups <= QIK_ATTN_WS_CTL_BYTES / 4) {
+      if (L->plan.ns > 2) L->fn = pick_kernel_d(a->D, fp16, vfp8, kv, Form::PIECES);
       L->grid = (int64_t)nx * std::min(sx, L->plan.wpx);
       L->ctl_bytes = QIK_ATTN_WS_CTL_BYTES;
       L->ws_bytes = L->ctl_bytes + (int64_t)L->plan.ngroups * L->plan.ns * L->slot;
