@@ -1183,6 +1183,8 @@ GemmPlan choose_plan(int64_t M, int64_t N, int64_t K, int cus) {
       const int64_t n1 = std::min(k * s1.bn, N);
       const int64_t t1 = cdiv(M, s1.bm) * cdiv(n1, s1.bn);
       const int64_t t2 = cdiv(M, s2.bm) * cdiv(N - n1, s2.bn);
+      // no order of the tiles ends before their total time shared by the CUs
+      if ((double)cdiv(t1, 8) * d1 + (double)cdiv(t2, 8) * d2 >= best_t * 0.97 * (double)P) continue;
       const double t = xcd_makespan(cdiv(t1, 8), d1, cdiv(t2, 8), d2, P);
       if (t < best_t * 0.97) {
         best_t = t;
