@@ -144,7 +144,7 @@ def block_causal_flash_attention(
 
     ``split_tail`` (keyword only, not in the reference): True (default) runs
     ``qik_attn_fwd_ws`` (resident workgroups pulling row blocks from per-XCD
-    queues, the last partial round's row blocks split in two over their KV
+    queues, the last partial round's row blocks split over their KV
     tiles) with a zeroed workspace kept per (device, stream); False runs
     ``qik_attn_fwd``, one workgroup per row block.
     """

@@ -1129,8 +1129,8 @@ inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 inline int64_t steps_of(int64_t K) { return cdiv(K, 128); }  // 128-k-byte steps
 
 // Finish time of one XCD whose P CUs run t1 tiles of time d1 and then t2
-// tiles of time d2, one workgroup per CU (a 256-thread workgroup of these
-// tiles holds a CU's four SIMDs), each started on the CU that frees first.
+// tiles of time d2, one workgroup per CU (a workgroup of these tiles holds
+// a CU's four SIMDs), each started on the CU that frees first.
 double xcd_makespan(int64_t t1, double d1, int64_t t2, double d2, int64_t P) {
   const int64_t full = t1 / P, rem = t1 % P;
   const double a = (double)full * d1, b = a + d1;  // CUs free after t1: P - rem at a, rem at b
