@@ -82,9 +82,12 @@ def _rms_rope_qk(query, key, norm_q, norm_k, freqs_cis):
     if query.dtype != key.dtype or query.shape[-1] != key.shape[-1] or query.device != key.device:
         return (fused_rms_norm_rope(query, norm_q.weight, freqs_cis, norm_q.eps),
                 fused_rms_norm_rope(key, norm_k.weight, freqs_cis, norm_k.eps))
+    # both entries are held here until the launch is enqueued: K's may clear Q's out
+    # of the cache, and with it the last references to the fp32 weight, cos and sin
+    # that Q's argument struct points to
+    ents = [_entry(x, norm.weight, freqs_cis, norm.eps) for x, norm in ((query, norm_q), (key, norm_k))]
     args, outs, reads = [], [], []
-    for x, norm in ((query, norm_q), (key, norm_k)):
-        ent = _entry(x, norm.weight, freqs_cis, norm.eps)
+    for x, ent in zip((query, key), ents):
         x = x.clone(memory_format=torch.contiguous_format) if ent.contig else x
         a = _lib.QikRmsRopeArgs.from_buffer_copy(ent.args)
         outs.append(x.new_empty(ent.shape))
