@@ -1212,7 +1212,12 @@ GemmPlan choose_plan(int64_t M, int64_t N, int64_t K, int cus) {
 // 5 slices against 15.9 in 8 slices of 128 x 128), 128 x 128 above.  At least
 // 48 steps, at most half the CUs' worth of tiles, and only when it is
 // estimated ahead of the unsplit plan with the second launch counted (about
-// 2.5 us, and the partials at about 5 TB/s).  slices = 1 means no split.
+// 2.5 us, and the partials at about 5 TB/s).  All slices of a tile run on one
+// XCD (fp8_gemm_split_kernel), so the fullest XCD has ceil(tiles / 8) * S of
+// them: S is limited to what its CUs run in one round, which is all that the
+// estimate counts (with cus / tiles slices, 33 to 36 on 32 CUs: 65 x 5376 x
+// 6144 20.2 us against 14.5, 129 x 5376 x 16384 44.3 against 30.9 unsplit).
+// slices = 1 means no split.
 struct KSplit {
   int slices, shape;
 };
@@ -1223,7 +1228,8 @@ KSplit choose_ksplit(int64_t M, int64_t N, int64_t K, int cus) {
   if (steps < 48) return {1, shape};
   const int64_t tiles = cdiv(M, kShapes[shape].bm) * cdiv(N, kShapes[shape].bn);
   if (tiles * 2 > cus) return {1, shape};
-  const int S = (int)std::min<int64_t>({cus / tiles, 8, steps / 8});
+  const int64_t P = std::max(1, cus / 8);
+  const int S = (int)std::min<int64_t>({P / cdiv(tiles, 8), 8, steps / 8});
   if (S < 2) return {1, shape};
   const double t_split = tile_time(shape, cdiv(steps, S)) + 2.5 + (double)(S * M * N) * 4.0 / 5e6;
   return {t_split < 0.95 * choose_plan(M, N, K, cus).t ? S : 1, shape};

@@ -430,6 +430,11 @@ def test_fp8_gemm_plan(mnk, plan, n1):
     ((40, 1040, 8208), [64, 64, 64, 64, 0, 8], 1040),
     ((64, 3072, 12288), [64, 64, 64, 64, 0, 5], 3072),
     ((65, 1040, 8208), [128, 128, 128, 128, 0, 8], 1040),
+    # the fullest XCD's share of the tiles times the slices fits its 32 CUs
+    ((65, 5376, 6144), [128, 128, 128, 128, 0, 5], 5376),      # 6 of 42 tiles: 5 slices, not 6
+    ((400, 1040, 8192), [128, 128, 128, 128, 0, 6], 1040),     # 5 of 36: 6, not 7
+    ((17, 5376, 6144), [64, 64, 64, 64, 0, 2], 5376),          # 11 of 84: 2, not 3
+    ((129, 5376, 16384), [64, 128, 64, 64, 0, 1], 0),          # 11 of 84 of 128 x 128: 2 do not pay
 ])
 def test_fp8_gemm_plan_tile_shapes(mnk, plan, n1):
     """Every tile shape and both K-split shapes are reached (256 CUs)."""
@@ -437,6 +442,25 @@ def test_fp8_gemm_plan_tile_shapes(mnk, plan, n1):
     n = ctypes.c_int64()
     assert _lib.load().qik_fp8_gemm_plan(*mnk, 0, got, ctypes.byref(n)) == 0
     assert list(got) == plan and n.value == n1
+
+
+def test_fp8_gemm_split_runs_in_one_round():
+    """No K split gives an XCD more workgroups than its CUs run at once (one each): the slices of
+    a tile all run on one XCD."""
+    lib = _lib.load()
+    got = (ctypes.c_int32 * 6)()
+    n = ctypes.c_int64()
+    split = 0
+    for cus in (256, 128, 304):
+        for K in (6144, 8192, 12288, 16384):
+            for N in range(256, 8193, 256):
+                for M in (1, 64, 65, 128, 129, 256, 257, 640):
+                    assert lib.qik_fp8_gemm_plan(M, N, K, cus, got, ctypes.byref(n)) == 0
+                    if got[5] > 1:
+                        split += 1
+                        tiles = -(-M // got[0]) * -(-N // got[1])
+                        assert -(-tiles // 8) * got[5] <= cus // 8, (M, N, K, cus, list(got))
+    assert split > 100
 
 
 def test_fp8_gemm_plan_checks():
