@@ -1098,24 +1098,27 @@ typedef CfgK128<128, 128, 2, 4, 3> Cfg128x128;
 typedef CfgK128<64, 128, 1, 4, 3> Cfg64x128;
 typedef CfgK128<64, 64, 2, 2, 4> Cfg64x64;
 
-// Time of a tile of each shape on a full chip, in us: t0 (prologue, output,
-// the launch's share) + t1 per 128-k-byte step.  Fitted to launches of one
-// round on MI355X, each shape forced (M x N x K 1728 x 9216 x 3072 43.9 us and
-// 4352 x 3072 x 12288 149.5 for 256 x 256; 1152 x 9216 x 3072 33.2, 3456 x
-// 3072 x 12288 135.5 for 192 x 256; 768 x 9216 x 3072 25.0, 1728 x 3072 x
+// Time of a tile of each shape, in us: t0 (prologue, output, the launch's share)
+// + t1 per 128-k-byte step.  Fitted to launches of one round on MI355X, each
+// shape forced, operands from memory (M x N x K 1728 x 9216 x 3072 43.9 us and
+// 4352 x 3072 x 12288 149.5 for 256 x 256; 768 x 9216 x 3072 25.0, 1728 x 3072 x
 // 12288 81.2 for 256 x 128; 2600 x 3072 x 3072 27.3, x 12288 87.3 for 128 x
 // 256; 1728 x 3072 x 3072 20.7, x 12288 69.7 for 192 x 128; 1152 x 3072 x 3072
 // 16.4, x 12288 51.7 for 128 x 128; 400 x 3072 x 3072 11.5, x 4096 x 4096 14.1
-// for 64 x 128; 203 x 3072 x 3072 8.9, x 4096 x 4096 11.1 for 64 x 64).  Over
-// 37 shapes of 64 to 4352 rows the plan they give was the fastest single shape
-// measured, or a mix, at every one.
+// for 64 x 128; 203 x 3072 x 3072 8.9, x 4096 x 4096 11.1 for 64 x 64) and, for
+// 192 x 256, after a quantiser (2075 x 4096 x 512 13.3 to 3456 x 3072 x 12288
+// 117.1: with 3.5 + 1.3 it won at 2 and 4 steps where 256 x 256 is faster, 4247
+// x 9216 x 256 39.1 against 34.6 with the quantiser, and lost at 96).  At 157 of 179 shapes of 64
+// to 4352 rows the plan they give is within 2% of the fastest of all tile shapes
+// and mixes measured there, on average 0.7% from it
+// (profiles/fp8_gemm_plan_candidates.md).
 struct TileShape {
   int bm, bn;
   double t0, t1;
 };
 enum { T256x256, T256x128, T128x128, T192x128, T192x256, T128x256, T64x128, T64x64, NSHAPES };
 static const TileShape kShapes[NSHAPES] = {{256, 256, 6.0, 1.5},   {256, 128, 6.0, 0.775}, {128, 128, 4.6, 0.485},
-                                           {192, 128, 4.6, 0.67},  {192, 256, 3.5, 1.3},   {128, 256, 6.0, 0.81},
+                                           {192, 128, 4.6, 0.67},  {192, 256, 4.5, 1.23},   {128, 256, 6.0, 0.81},
                                            {64, 128, 3.8, 0.32},   {64, 64, 3.8, 0.215}};
 // the (big, small) shape pairs a launch can take, as indices into kShapes
 // (both of a pair have the same number of waves)
@@ -1160,21 +1163,38 @@ double xcd_makespan(int64_t t1, double d1, int64_t t2, double d2, int64_t P) {
 struct GemmPlan {
   int pair;  // index into kPairs
   int64_t n1;
-  double t;  // estimated makespan, us
+  double t;  // makespan from the tile times, us
   bool small_first;  // launch the small tiles' region first (fp8_gemm_kernel)
 };
 
-// The split with the shortest estimated makespan on `cus` CUs.  Workgroups go
+// Estimated time of a launch whose busiest XCD of P CUs has `work` of tile time
+// and ends after `t`.  From 24 steps (K = 3072) on the matrix cores run long
+// enough that the clock follows the load: the tile times hold with three quarters of the CUs
+// busy, and with all of them busy a tile takes 14% longer.  (Quantiser + GEMM,
+// the weights of six layers in turn: time / makespan from the tile times, the
+// median over 1100 launches of 1000 to 4352 rows with each plan forced, 0.90 at
+// 0.55 to 0.65 of the CUs busy, 0.96 at 0.75, 0.98 at 0.85, 1.02 at 0.95, 1.05
+// at 1; at 2 to 12 steps 1.12 to 1.20 with no trend.)  Without it nearly full
+// mixes of smaller tiles win against fewer large ones that are faster: 4096 x
+// 3072 x 12288 (M x N x K) 143.8 us with 512 tiles of 256 x 128 and 128 x 128,
+// 137.3 with 192 of 256 x 256; 3456 x 3072 x 12288 130.2 and 117.1 (192 x 256).
+constexpr int64_t LONG_STEPS = 24;
+inline double launch_time(double t, double work, int64_t P, int64_t steps) {
+  return steps < LONG_STEPS ? t : t * (1.0 + 0.55 * std::max(0.0, work / (t * (double)P) - 0.75));
+}
+
+// The split with the shortest estimated time on `cus` CUs.  Workgroups go
 // to the XCDs in turn, so the XCD that finishes last holds ceil(tiles / 8) of
 // each region.  The split points are whole big-tile columns; n1 = N is one
 // region of the big shape, n1 = 0 one of the small shape.  A later candidate
-// replaces an earlier one only if it is estimated 3% faster (the times above
-// are good to a few percent); the first candidate is 256 x 256 tiles.
+// replaces an earlier one only if it is estimated faster by what the estimate
+// is good to (1%; 3% below LONG_STEPS); the first candidate is 256 x 256 tiles.
 GemmPlan choose_plan(int64_t M, int64_t N, int64_t K, int cus) {
   const int64_t P = std::max(1, (cus > 0 ? cus : 256) / 8);
-  GemmPlan best = {0, N, 0.0};
+  GemmPlan best = {0, N, 0.0, false};
   double best_t = 1e300;
   const int64_t steps = steps_of(K);
+  const double ahead = steps < LONG_STEPS ? 0.97 : 0.99;
   for (int pr = 0; pr < NPAIRS; ++pr) {
     const TileShape& s1 = kShapes[kPairs[pr][0]];
     const TileShape& s2 = kShapes[kPairs[pr][1]];
@@ -1184,15 +1204,16 @@ GemmPlan choose_plan(int64_t M, int64_t N, int64_t K, int cus) {
       const int64_t t1 = cdiv(M, s1.bm) * cdiv(n1, s1.bn);
       const int64_t t2 = cdiv(M, s2.bm) * cdiv(N - n1, s2.bn);
       // no order of the tiles ends before their total time shared by the CUs
-      if ((double)cdiv(t1, 8) * d1 + (double)cdiv(t2, 8) * d2 >= best_t * 0.97 * (double)P) continue;
+      const double work = (double)cdiv(t1, 8) * d1 + (double)cdiv(t2, 8) * d2;
+      if (work >= best_t * ahead * (double)P) continue;
       const double t = xcd_makespan(cdiv(t1, 8), d1, cdiv(t2, 8), d2, P);
-      if (t < best_t * 0.97) {
-        best_t = t;
+      const double est = launch_time(t, work, P, steps);
+      if (est < best_t * ahead) {
+        best_t = est;
         best = {pr, n1, t, false};
       }
     }
   }
-  best.t = best_t;
   // the small tiles first when that is estimated no slower (measured: 1-2%
   // faster at 4352 x 9216 x 3072 and 4352 x 12288 x 3072, whose makespans are
   // equal either way; 12% slower at 1543 x 9232 x 1104, whose is not)
@@ -1202,7 +1223,7 @@ GemmPlan choose_plan(int64_t M, int64_t N, int64_t K, int cus) {
   const int64_t t2 = cdiv(M, s2.bm) * cdiv(N - best.n1, s2.bn);
   if (t1 > 0 && t2 > 0)
     best.small_first = xcd_makespan(cdiv(t2, 8), tile_time(kPairs[best.pair][1], steps), cdiv(t1, 8),
-                                    tile_time(kPairs[best.pair][0], steps), P) <= best_t * 1.0001;
+                                    tile_time(kPairs[best.pair][0], steps), P) <= best.t * 1.0001;
   return best;
 }
 

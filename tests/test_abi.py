@@ -435,6 +435,14 @@ def test_fp8_gemm_plan(mnk, plan, n1):
     ((400, 1040, 8192), [128, 128, 128, 128, 0, 6], 1040),     # 5 of 36: 6, not 7
     ((17, 5376, 6144), [64, 64, 64, 64, 0, 2], 5376),          # 11 of 84: 2, not 3
     ((129, 5376, 16384), [64, 128, 64, 64, 0, 1], 0),          # 11 of 84 of 128 x 128: 2 do not pay
+    # a long launch's clock falls with the CUs it keeps busy: fewer, larger tiles
+    ((4096, 3072, 12288), [256, 256, 256, 128, 0, 1], 3072),   # not 512 of 256 x 128 and 128 x 128
+    ((3456, 3072, 12288), [192, 256, 192, 128, 0, 1], 3072),
+    ((2075, 4096, 4096), [192, 256, 192, 128, 0, 1], 4096),
+    ((2900, 12288, 3072), [256, 256, 256, 128, 1, 1], 10752),
+    # two and four steps: 192 x 256 is not the cheapest
+    ((4247, 9216, 256), [256, 256, 256, 128, 1, 1], 7680),
+    ((1842, 4096, 512), [256, 256, 256, 128, 0, 1], 0),
 ])
 def test_fp8_gemm_plan_tile_shapes(mnk, plan, n1):
     """Every tile shape and both K-split shapes are reached (256 CUs)."""
