@@ -173,10 +173,11 @@ int qik_attn_fwd_noalloc(const qik_attn_args* args, void* stream);
  * when item/piece/group are not NULL (cap >= grid entries each), per
  * workgroup (or, for qik_attn_fwd_ws, queue position loc of XCD x at index
  * loc * 8 + x): its row block (-1: no work), its piece and its workspace
- * group (-1: not split).  The other pieces of a row block with few KV tiles
- * (fewer than 16, four per piece when there are more than two) are skipped on
- * the device (the first runs the whole row block).  Launches at D = 256
- * keep two pieces where this map has four or eight.
+ * group (-1: not split).  The device cuts a row block with few KV tiles into
+ * fewer pieces and skips the others: eight pieces become four below 32 tiles,
+ * and a row block runs whole below 16 (below 8 in the launches of at most half
+ * a row block per CU).  Launches at D = 256 keep two pieces where this map has
+ * four or eight.
  * `split` = 0 gives qik_attn_fwd's assignment.  This form assumes the 8 XCDs
  * of an MI355X; the launches use the XCD count the device reports. */
 int qik_attn_work_map(int64_t n_items, int32_t n_row_blocks, int32_t slots_per_xcd, int32_t split,

@@ -102,8 +102,12 @@ struct Params {
 // and piece 1 the rest.
 constexpr int SPLIT_MIN_TILES = 16;
 // An item of four or eight pieces (a nearly empty last round, qik_plan.h) is
-// cut into equal ones, and runs whole below four tiles a piece.
+// cut into equal ones of at least four tiles: into four where eight would be
+// shorter (2 x 24 heads x 1408 rows, 16 left-over row blocks of 22 tiles: 61.5
+// us in four, 64.2 in two, 71.5 whole; x 1344 58.7 / 60.8 / 67.0).
 constexpr int MANY_MIN_TILES = 4;
+constexpr int MANY_FEWER = 4;
+static_assert(SPLIT_MIN_TILES >= MANY_MIN_TILES * MANY_FEWER, "a split item has the tiles for the fewer pieces");
 // The two-group kernel splits more finely: its launches leave most of the
 // device idle, so a piece or a group is worth having wherever it saves more
 // than its merge.  Two groups merge in LDS (about 1 us) from 4 tiles on, two
@@ -588,14 +592,16 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
       run1 = (Lmax >= s1) ? min(cdiv_i(p.SN, BN), (Lmax - s1) / BN + 1) : 0;
     };
     bool gsplit_on = false;  // two-group kernel: the unit's tiles are split between the groups
+    [[maybe_unused]] int ns = p.plan.ns;  // many pieces: those of this item
     auto piece_tiles = [&](int T, int& g0, int& g1) {
-      // this unit's tiles [g0, g1): all of them, or one of the item's two
-      // pieces (T, and so the split, is the same for both pieces of the item)
+      // this unit's tiles [g0, g1): all of them, or one of the item's pieces;
+      // true for a piece (T, and so the split, is the same for all of the
+      // item's; those past the number it is cut into are not run)
       bool split = wk.group >= 0 && T >= (KSPLIT == 1 ? SPLIT_MIN_TILES : PIECE_MIN_TILES);
       if constexpr (KSPLIT == 1) {
-        [[maybe_unused]] const int ns = p.plan.ns;
         if (MANY) {
-          split = split && T >= MANY_MIN_TILES * ns;
+          if (T < MANY_MIN_TILES * ns) ns = MANY_FEWER;
+          split = split && wk.piece < ns;
           g0 = split ? T * wk.piece / ns : 0;
           g1 = split ? T * (wk.piece + 1) / ns : T;
         } else {
@@ -912,7 +918,7 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
       // it back).  A piece that finds the other one already arrived merges
       // at once and never writes its own slot; otherwise it publishes its
       // slot and arrives, and the second to arrive merges.
-      const unsigned others = MANY ? (unsigned)(pe.plan.ns - 1) : 1u;
+      const unsigned others = MANY ? (unsigned)(ns - 1) : 1u;
       if (lead) sred[0][0] = g_load(word) == others ? 1 : 0;
       __syncthreads();
       const bool other_first = sred[0][0] != 0;
@@ -957,7 +963,6 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
         // which piece merges.  Half of the accumulators per pass: with all of
         // them the merge needs three sets of 64 registers and the kernel spills
         // 16 to 30 (2 x 24 heads x 2772 rows 359.3 us, 355.2 with halves).
-        const int ns = pe.plan.ns;
         float mm = m_run;
         for (int pc = 0; pc < ns; ++pc) {
           if (pc == wk.piece) continue;

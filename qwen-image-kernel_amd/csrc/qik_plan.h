@@ -76,10 +76,13 @@ QIK_HD inline int plan_full(int q, int sx) { return q >= sx ? sx * (q / sx) : 0;
 // sixth of the slots, eight when at most a sixteenth: two pieces would leave
 // the CUs idle for most of a piece's time (2 x 24 heads x 2772 rows against
 // 4907 keys, 4 row blocks of 132 per XCD left over: 394 us with two pieces, 375
-// with four, 371 with eight; 2 x 24 x 2700 against 3500 265 / 257 / 256).  More
-// pieces cost their merge, one slot after the other (about 4 us each), so a
-// fuller round keeps two (four and eight pieces of a half-full round: 351 and
-// 378 us against 345).
+// with four, 371 with eight; 2 x 24 x 2700 against 3500 265 / 257 / 256).  Eight
+// against four is worth most with few left over and many tiles (16 heads x 4224
+// rows, 2 per XCD: 141.5 us with eight, 144.8 with four, fp16 with a key mask
+// 160.1 / 167.2; 12 x 5760, 4 per XCD: 209.7 / 213.7) and is never slower there.
+// More pieces cost their merge, one slot after the other (about 4 us each), so
+// a fuller round keeps two (four and eight pieces of a half-full round: 351 and
+// 378 us against 345).  The kernel cuts a row block with few tiles into fewer.
 inline int plan_pieces(int r, int sx, bool rounds) {
   if (r <= 0) return 1;
   if (rounds && r * 16 <= sx) return MAX_PIECES;

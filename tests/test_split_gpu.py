@@ -214,7 +214,7 @@ def test_split_decode_against_fp8_slab(H):
 @pytest.mark.parametrize("H,D,rows,keys,pieces,dtype", [
     (65, 128, 1024, 2100, 8, torch.bfloat16),   # 65 row blocks per XCD: one left over, 33 tiles in 8 pieces
     (65, 128, 1024, 2000, 8, torch.bfloat16),   # 32 tiles: the fewest that 8 pieces take
-    (65, 128, 1024, 1970, 8, torch.float16),    # 31 tiles: the left-over row blocks run whole
+    (65, 128, 1024, 1970, 8, torch.float16),    # 31 tiles: four of the 8 pieces
     (72, 128, 1000, 1100, 4, torch.bfloat16),   # 72 per XCD: 8 left over, 18 tiles in 4 pieces
     (97, 64, 1000, 2500, 8, torch.bfloat16),    # D = 64, three workgroups per CU: 97 row blocks on 96 slots
 ])
@@ -248,6 +248,46 @@ def test_nearly_empty_last_round(H, D, rows, keys, pieces, dtype):
     ref = oa.attention_fp32(*sel, L)
     _check(outs[0][:, :, heads], ref, f"last round H={H}")
     assert (outs[0][:, 7] == 0).all()
+
+
+@pytest.mark.parametrize("keys,pieces", [
+    (2112, 8),   # 33 tiles
+    (1985, 8),   # 32: the fewest that eight pieces take
+    (1984, 4),   # 31
+    (1408, 4),   # 22
+    (961, 4),    # 16: the fewest that are cut at all
+    (960, 1),    # 15: whole
+])
+@pytest.mark.parametrize("uniform", [False, True])
+def test_left_over_row_blocks_are_cut_by_their_tiles(keys, pieces, uniform):
+    """One row block per XCD left over after a whole round (a plan of eight pieces): the
+    pieces that publish their state are those the row block's KV tiles allow (all of
+    them, or all but the last to finish), the other slots stay untouched, and the
+    result is the unsplit launch's."""
+    if _cus() != 256:
+        pytest.skip("the shape leaves one row block per XCD on 256 CUs")
+    _flush(f"case pieces by tiles keys={keys} uniform={uniform}")
+    H, D, rows = 65, 128, 1024
+    g = torch.Generator(device=DEV).manual_seed(70 + keys)
+    q = torch.randn(1, rows, H, D, generator=g, device=DEV).to(torch.bfloat16)
+    k, v = (torch.randn(1, keys, H, D, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    L = None if uniform else torch.full((rows,), keys - 1, dtype=torch.int32, device=DEV)
+    out = torch.empty_like(q)
+    args = make_args(q, k, v, L, None, out, None, None, None, uniform)
+    nbytes = _ws_bytes(args)
+    slot = 128 * D * 4 + 2048
+    assert nbytes == _lib.WS_CTL_BYTES + 8 * 8 * slot   # 8 groups of 8 slots
+    ws = torch.zeros(nbytes, dtype=torch.uint8, device=DEV)
+    ws[_lib.WS_CTL_BYTES:] = 0xEE
+    _lib.check(_lib.load().qik_attn_fwd_ws(ctypes.byref(args), ws.data_ptr(), nbytes,
+                                           torch.cuda.current_stream().cuda_stream), "qik_attn_fwd_ws")
+    torch.cuda.synchronize()
+    assert (ws[:_lib.WS_CTL_BYTES] == 0).all()
+    written = (ws[_lib.WS_CTL_BYTES:].view(8, 8, slot) != 0xEE).any(-1).sum(-1).tolist()
+    assert all(n in ((0,) if pieces == 1 else (pieces - 1, pieces)) for n in written), written
+    plain = qik.block_causal_flash_attention(q, k, v, L, None, uniform_full=uniform, split_tail=False)
+    d = (out.float() - plain.float()).abs()
+    assert d.max().item() <= 2 * MAX_ABS and d.mean().item() <= 5e-4
 
 
 @pytest.mark.parametrize("keys", [64, 129, 250, 257, 449, 512, 575, 960, 1000])
