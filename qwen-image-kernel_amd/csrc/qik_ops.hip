@@ -212,12 +212,19 @@ __device__ __forceinline__ void rms_rope_rows(const RmsRopeParams& p, const int 
   }
 }
 
+template <int D, bool FP16>
+__global__ void __launch_bounds__(NTHREADS) rms_rope_kernel(const RmsRopeParams p) {
+  rms_rope_rows<D, FP16>(p, (int)blockIdx.x);
+}
+
 // Workgroups [0, na) take a's rows, the others b's (a layer's Q and K in one
 // launch: at 1728 x 24 x 128 each of two launches took 6.8 us, half of that its
-// own start and end; the whole layer 151.1 -> 146.3 us with one).
+// own start and end; the whole layer 151.1 -> 146.3 us with one).  A kernel of
+// its own: choosing between two parameter sets costs a single call 0.1 to 0.3
+// of 4 us (300 x 4 x 64 4.36 us against 4.11, 500 x 24 x 32 3.82 against 3.56).
 template <int D, bool FP16>
-__global__ void __launch_bounds__(NTHREADS) rms_rope_kernel(const RmsRopeParams a, const RmsRopeParams b,
-                                                            const int na) {
+__global__ void __launch_bounds__(NTHREADS) rms_rope_pair_kernel(const RmsRopeParams a, const RmsRopeParams b,
+                                                                 const int na) {
   const bool first = (int)blockIdx.x < na;
   rms_rope_rows<D, FP16>(first ? a : b, (int)blockIdx.x - (first ? 0 : na));
 }
@@ -598,18 +605,24 @@ int prepare_rope(const qik_rms_rope_args* a, RmsRopeParams* p, int64_t* grid) {
   return QIK_OK;
 }
 
-int launch_rope(int64_t D, bool fp16, RmsRopeParams& a, int64_t ga, RmsRopeParams& b, int64_t gb, void* stream) {
+// One call (b NULL) or both in one launch.
+int launch_rope(int64_t D, bool fp16, RmsRopeParams& a, int64_t ga, RmsRopeParams* b, int64_t gb, void* stream) {
   if (ga + gb == 0) return QIK_OK;
   if (ga + gb > (int64_t)INT_MAX) return QIK_ERR_SHAPE;
-  const void* const fns[4][2] = {
-      {(const void*)rms_rope_kernel<32, false>, (const void*)rms_rope_kernel<32, true>},
-      {(const void*)rms_rope_kernel<64, false>, (const void*)rms_rope_kernel<64, true>},
-      {(const void*)rms_rope_kernel<128, false>, (const void*)rms_rope_kernel<128, true>},
-      {(const void*)rms_rope_kernel<256, false>, (const void*)rms_rope_kernel<256, true>}};
+  const void* const fns[4][2][2] = {
+      {{(const void*)rms_rope_kernel<32, false>, (const void*)rms_rope_kernel<32, true>},
+       {(const void*)rms_rope_pair_kernel<32, false>, (const void*)rms_rope_pair_kernel<32, true>}},
+      {{(const void*)rms_rope_kernel<64, false>, (const void*)rms_rope_kernel<64, true>},
+       {(const void*)rms_rope_pair_kernel<64, false>, (const void*)rms_rope_pair_kernel<64, true>}},
+      {{(const void*)rms_rope_kernel<128, false>, (const void*)rms_rope_kernel<128, true>},
+       {(const void*)rms_rope_pair_kernel<128, false>, (const void*)rms_rope_pair_kernel<128, true>}},
+      {{(const void*)rms_rope_kernel<256, false>, (const void*)rms_rope_kernel<256, true>},
+       {(const void*)rms_rope_pair_kernel<256, false>, (const void*)rms_rope_pair_kernel<256, true>}}};
   int na = (int)ga;
-  void* kargs[] = {&a, &b, &na};
-  const hipError_t e = hipLaunchKernel(fns[head_dim_index(D)][fp16 ? 1 : 0], dim3((unsigned)(ga + gb)),
-                                       dim3(NTHREADS), kargs, 0, static_cast<hipStream_t>(stream));
+  void* one[] = {&a};
+  void* both[] = {&a, b, &na};
+  const hipError_t e = hipLaunchKernel(fns[head_dim_index(D)][b != nullptr][fp16 ? 1 : 0], dim3((unsigned)(ga + gb)),
+                                       dim3(NTHREADS), b != nullptr ? both : one, 0, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? QIK_OK : QIK_ERR_LAUNCH;
 }
 
@@ -623,7 +636,7 @@ int qik_rms_rope(const qik_rms_rope_args* a, void* stream) {
   int64_t grid = 0;
   const int st = prepare_rope(a, &p, &grid);
   if (st != QIK_OK) return st;
-  return launch_rope(a->D, a->dtype == QIK_DTYPE_FP16, p, grid, p, 0, stream);
+  return launch_rope(a->D, a->dtype == QIK_DTYPE_FP16, p, grid, nullptr, 0, stream);
 }
 
 int qik_rms_rope_pair(const qik_rms_rope_args* a, const qik_rms_rope_args* b, void* stream) {
@@ -635,7 +648,7 @@ int qik_rms_rope_pair(const qik_rms_rope_args* a, const qik_rms_rope_args* b, vo
   if (st != QIK_OK) return st;
   if (a->D != b->D) return QIK_ERR_HEAD_DIM;
   if (a->dtype != b->dtype) return QIK_ERR_DTYPE;
-  return launch_rope(a->D, a->dtype == QIK_DTYPE_FP16, pa, ga, pb, gb, stream);
+  return launch_rope(a->D, a->dtype == QIK_DTYPE_FP16, pa, ga, &pb, gb, stream);
 }
 
 }  // extern "C"
