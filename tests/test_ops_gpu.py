@@ -150,6 +150,12 @@ def test_slab_store_row_steps(P, D, v_fp8):
     (1, 2731, 24, 64, True),
     (1, 5462, 24, 128, False),  # four rows per copy thread
     (1, 5461, 3, 32, False),    # one
+    (1, 425, 24, 128, True),    # fp8, small V: one row per copy thread
+    (1, 427, 24, 128, True),    # four, from here on
+    (4, 33, 96, 128, True),     # four, the row step longer than a prefix
+    (2, 110, 96, 64, True),
+    (3, 31, 100, 256, True),
+    (2, 700, 64, 32, True),
 ])
 def test_slab_store_launch_forms(B, P, H, D, v_fp8):
     """Both sides of each line between the store's launch forms, through the workspace
