@@ -751,10 +751,11 @@ int store(const qik_slab_store_args* a, float* partial, hipStream_t s) {
     // extra ones find no row), so the codes launch re-reads its V rows from the
     // L2 that the scale launch read them through.  K goes with the codes from
     // LARGE_V bytes of V on: the codes' blocks alone are too short a launch to
-    // fill the memory's time there (V of 15.7 MB 14.3 us against 15.7 with K
-    // beside the scales, 51 MB 30.0 / 32.7; below, the scales alone are the
-    // short launch: 4.3 MB 10.3 / 9.2, 4.6 MB 10.3 / 9.3).
-    constexpr int64_t LARGE_V = 8 << 20;
+    // fill the memory's time there (K beside the scales / beside the codes, 24
+    // heads x 128: V of 9.2 MB 11.5 / 12.0 us, 10.8 12.6 / 12.7, 12.6 13.9 / 13.4,
+    // 16.0 16.3 / 14.7, 21.5 20.0 / 18.1; 24 x 64 10.8 12.6 / 12.8, 12.3 13.5 /
+    // 13.3; 4 to 12 heads cross a little later, 12.3 MB 14.7 / 15.1).
+    constexpr int64_t LARGE_V = 11 << 20;
     const bool large = threads * 16 >= LARGE_V;
     // four rows per copy thread from five copy workgroups of one row a thread for
     // every four CUs on (V of 3.1 MB 8.14 us against 8.45 with one, 1.8 MB 7.21 /

@@ -143,8 +143,11 @@ def test_slab_store_row_steps(P, D, v_fp8):
 
 
 @pytest.mark.parametrize("B,P,H,D,v_fp8", [
-    (1, 1365, 24, 128, True),   # V just below 8 MiB: K copied beside the scales
-    (1, 1366, 24, 128, True),   # just above: beside the codes
+    (1, 1365, 24, 128, True),   # V around 8 MiB: K copied beside the scales
+    (1, 1366, 24, 128, True),
+    (1, 1877, 24, 128, True),   # V just below 11 MiB: the same
+    (1, 1878, 24, 128, True),   # just above: beside the codes
+    (1, 3755, 24, 64, True),
     (2, 1400, 12, 128, True),
     (1, 2730, 24, 64, True),
     (1, 2731, 24, 64, True),
