@@ -166,9 +166,12 @@ class _LayerView:
         """``buf[layer, :, :, :P, :].transpose(1, 2)`` in one view op (1.7 us of host time for
         the chain's 5.6, of which a store and its views have two)."""
         sl, sb, sh, sp, sd = buf.stride()
-        _, B, H, cap, D = buf.shape
+        n, B, H, cap, D = buf.shape
+        i = self._layer
+        if not -n <= i < n:  # as_strided checks the storage only, and takes no negative index
+            raise IndexError(f"layer {i} is out of range for a slab of {n} layers")
         return buf.as_strided((B, P if P < cap else cap, H, D), (sb, sp, sh, sd),
-                              buf.storage_offset() + self._layer * sl)
+                              buf.storage_offset() + (i if i >= 0 else i + n) * sl)
 
     def views(self):
         """(k, v, v_scale_or_None) for block_causal_flash_attention."""

@@ -556,6 +556,27 @@ def test_slab_views_are_the_indexed_views(P):
             assert got.untyped_storage().data_ptr() == buf.untyped_storage().data_ptr()
 
 
+def test_slab_views_take_the_layers_that_indexing_takes():
+    """A view of layer -1 reads the last layer, also of a slab that is part of a larger
+    buffer; a layer past the slab raises IndexError rather than reading its neighbours."""
+    import torch
+    import qwen_image_kernel_amd as qik
+    from qwen_image_kernel_amd.kv_cache import _LayerView
+    g = torch.Generator().manual_seed(8)
+    cache = qik.ContiguousKVCache(3, 2, 16, 4, 32, v_fp8=False, device="cpu")
+    cache.get_layer(2).store(*(torch.randn(2, 9, 4, 32, generator=g).to(torch.bfloat16) for _ in range(2)))
+    big = torch.randn(5, 2, 4, 16, 32, generator=g).to(torch.bfloat16)
+    for k_buf in (cache.k_buf, big[1:4]):
+        cache.k_buf = k_buf
+        assert torch.equal(_LayerView(cache, -1).get()[0], k_buf[-1, :, :, :9, :].transpose(1, 2))
+        for layer in (3, -4):
+            with pytest.raises(IndexError):
+                _LayerView(cache, layer).get()
+    cache.k_buf = big[1:3]
+    with pytest.raises(IndexError):
+        cache.get_layer(2).views()
+
+
 @pytest.mark.parametrize("v_fp8", [False, True])
 def test_cpu_slab_takes_any_float_dtype_like_the_reference(v_fp8):
     """A CPU slab is stored by the reference's torch ops (kv_cache.py:30-45),
