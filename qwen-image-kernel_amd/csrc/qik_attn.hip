@@ -107,7 +107,9 @@ constexpr int SPLIT_MIN_TILES = 16;
 // us in four, 64.2 in two, 71.5 whole; x 1344 58.7 / 60.8 / 67.0).
 constexpr int MANY_MIN_TILES = 4;
 constexpr int MANY_FEWER = 4;
+constexpr int FEWER_FLAG = 16;  // in Work::piece, through the tile loop: cut into MANY_FEWER
 static_assert(SPLIT_MIN_TILES >= MANY_MIN_TILES * MANY_FEWER, "a split item has the tiles for the fewer pieces");
+static_assert(MAX_PIECES <= FEWER_FLAG, "piece indexes stay below the flag");
 // The two-group kernel splits more finely: its launches leave most of the
 // device idle, so a piece or a group is worth having wherever it saves more
 // than its merge.  Two groups merge in LDS (about 1 us) from 4 tiles on, two
@@ -592,7 +594,6 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
       run1 = (Lmax >= s1) ? min(cdiv_i(p.SN, BN), (Lmax - s1) / BN + 1) : 0;
     };
     bool gsplit_on = false;  // two-group kernel: the unit's tiles are split between the groups
-    [[maybe_unused]] int ns = p.plan.ns;  // many pieces: those of this item
     auto piece_tiles = [&](int T, int& g0, int& g1) {
       // this unit's tiles [g0, g1): all of them, or one of the item's pieces;
       // true for a piece (T, and so the split, is the same for all of the
@@ -600,7 +601,7 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
       bool split = wk.group >= 0 && T >= (KSPLIT == 1 ? SPLIT_MIN_TILES : PIECE_MIN_TILES);
       if constexpr (KSPLIT == 1) {
         if (MANY) {
-          if (T < MANY_MIN_TILES * ns) ns = MANY_FEWER;
+          const int ns = T < MANY_MIN_TILES * p.plan.ns ? MANY_FEWER : p.plan.ns;
           split = split && wk.piece < ns;
           g0 = split ? T * wk.piece / ns : 0;
           g1 = split ? T * (wk.piece + 1) / ns : T;
@@ -655,6 +656,9 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
     int g0, g1;
     const bool split = piece_tiles(T, g0, g1);
     if (wk.piece > 0 && !split) continue;
+    // (not a variable of its own: one more value live through the tile loop made
+    // the D = 64 kernel 3.5% slower, 2 x 24 heads x 4200 rows 252.5 us against 243.3)
+    if (MANY && T < MANY_MIN_TILES * p.plan.ns) wk.piece |= FEWER_FLAG;
 
     // ---- LDS operand offsets inside a stage (lane constants)
     const int swk = swz<CH>(l32);  // rows l32 and l32 + 32 share it
@@ -909,6 +913,8 @@ __global__ void __launch_bounds__(NTHREADS * KSPLIT, (KSPLIT == 1 && D <= 128) ?
     }
     float l_part = l_run;
     if (split) {
+      [[maybe_unused]] const int ns = (wk.piece & FEWER_FLAG) ? MANY_FEWER : pe.plan.ns;  // the item's pieces
+      if (MANY) wk.piece &= FEWER_FLAG - 1;
       constexpr int OB = slot_oacc_bytes<D>();
       constexpr int SB = slot_bytes<D>();
       constexpr int SC1 = 16;  // cache policy: device scope
