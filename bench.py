@@ -763,7 +763,8 @@ def main():
             "kernel": f"attn_fwd_kernel ({dom})",
             "launch": ("qik_attn_fwd_ws: one workgroup per resident slot (2 per CU) pulling row "
                        "blocks from per-XCD queues; the last partial round's row blocks split in two "
-                       "pieces (7/10 and 3/10 of their KV tiles) merged through the workspace"),
+                       "pieces (7/10 and 3/10 of their KV tiles; four or eight equal ones when that "
+                       "round is nearly empty) merged through the workspace"),
             "achieved": round(achieved, 2),
             "launch_timing": "HIP events around each launch of the last timed step, on the launch stream",
             "peak": PEAK_BF16_TFLOPS,

@@ -82,7 +82,7 @@ typedef struct qik_slab_store_args {
   int64_t stride_v[3];        /* b, p, h of v                                        */
   int64_t stride_k_dst[3];    /* b, h, p of k_dst                                    */
   int64_t stride_v_dst[3];    /* b, h, p of v_dst                                    */
-  int64_t* length_dst;        /* optional: the store's first launch also writes P
+  int64_t* length_dst;        /* optional: the launch that copies K also writes P
                                  here (the layer's entry of a device length table,
                                  kv_cache.py:45 sets it after the store); NULL: not
                                  written.  Nothing is launched, and nothing written,
@@ -91,8 +91,9 @@ typedef struct qik_slab_store_args {
 
 int qik_slab_store(const qik_slab_store_args* args, void* stream);
 
-/* The same store in two launches instead of three, for an fp8 V: the K copy and
- * the scales of the V rows' chunks in one launch, the codes in the second
+/* The same store in two launches instead of three, for an fp8 V: the scales of
+ * the V rows' chunks in the first launch, the codes in the second, the K copy
+ * beside the scales (V below 11 MiB) or the codes
  * (replaces the body of _LayerView.store, kv_cache.py:30-45, like
  * qik_slab_store; the results are bit-identical to it).  The chunks' scales
  * go to the caller's workspace, at least qik_slab_store_workspace_size bytes,

@@ -20,9 +20,10 @@
 // = activation rows m), so each lane ends with 4 consecutive n of one row m
 // per register quad.  Tiles of A and W reach LDS directly
 // (buffer_load_dwordx4 ... lds, no register staging), 128 k-bytes per stage,
-// two to four stages ahead of their use, with a 16-byte chunk swizzle that
-// makes the fragment reads conflict-free; each wave reads the next fragments while its
-// MFMAs run on the current ones, and the copies are issued between the MFMAs.
+// one to three stages ahead of their use, with a 16-byte chunk swizzle that
+// makes the fragment reads conflict-free; each wave reads the next fragments
+// while its MFMAs run on the current ones, and the copies are issued between
+// the MFMAs.
 // The outputs go out through LDS as whole rows.  Workgroups map to tiles XCD
 // by XCD (the dispatcher deals workgroup b to XCD b % 8), so one XCD's L2
 // serves a compact block of tiles.
@@ -529,7 +530,7 @@ struct GemmParams {
 
 // Tile shape BM x BN, NS stages of 128 k-bytes (two MFMA k-steps per barrier;
 // each copied row a whole 128-byte line), WGM x WGN waves.  A stage's copies go
-// out NS steps ahead of its first fragment reads.
+// out NS - 1 steps ahead of its first fragment reads.
 //
 // What bounds a tile of the smaller shapes is the latency of those copies: at
 // two stages a step cannot be shorter than one L2 or HBM round trip (about
@@ -1205,7 +1206,7 @@ GemmPlan choose_plan(int64_t M, int64_t N, int64_t K, int cus) {
       const int64_t t2 = cdiv(M, s2.bm) * cdiv(N - n1, s2.bn);
       // no order of the tiles ends before their total time shared by the CUs
       const double work = (double)cdiv(t1, 8) * d1 + (double)cdiv(t2, 8) * d2;
-      if (work >= best_t * ahead * (double)P) continue;
+      if (launch_time(work / (double)P, work, P, steps) >= best_t * ahead) continue;
       const double t = xcd_makespan(cdiv(t1, 8), d1, cdiv(t2, 8), d2, P);
       const double est = launch_time(t, work, P, steps);
       if (est < best_t * ahead) {

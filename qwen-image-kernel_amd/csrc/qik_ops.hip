@@ -243,7 +243,7 @@ struct CopyParams {
   int64_t rows;      // B*H*P
   int64_t P, H;
   int row_bytes;     // D * element size
-  int64_t* len_dst;  // NULL, or where the first launch writes P
+  int64_t* len_dst;  // NULL, or where the launch that copies K writes P
 };
 
 // CR passes of THREADS / (row_bytes / 16) rows per workgroup, their loads issued

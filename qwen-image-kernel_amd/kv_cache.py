@@ -51,7 +51,7 @@ class _LayerView:
         if P > c.capacity:
             raise ValueError(f"prefix of {P} tokens exceeds the slab capacity {c.capacity}")
         if c.k_buf.is_cuda and P > 0 and k.shape[0] > 0 and k.shape[2] > 0:
-            # the store's first launch also writes lengths[layer] = P
+            # the store's launch that copies K also writes lengths[layer] = P
             self._store_device(k, v, P)
         else:
             if c.k_buf.is_cuda:
