@@ -526,7 +526,7 @@ def side_ops(qik, wls, dev, with_cpu: bool) -> dict:
     api_us, host_us = _batch_us(api, 50), _host_us(api, 200)
     nbytes = B * P * H * D * (2 + 2 + 2 + 1) + B * H * 4   # k, v in; k bf16, v fp8 out; scales
     entry = {"shape": [B, P, H, D],
-             "kernels": "slab_copy_scale_kernel<128> + slab_quant_fp8_kernel<128> (qik_slab_store_ws)",
+             "kernels": "slab_partial_scale_kernel<128> + slab_quant_copy_kernel<128> (qik_slab_store_ws)",
              "us": round(us, 2), "api_us": round(api_us, 2), "host_us": round(host_us, 2),
              "algorithmic_bytes": nbytes,
              "us_three_launch_form": round(us3, 2),

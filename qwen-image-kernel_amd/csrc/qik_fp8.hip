@@ -1211,16 +1211,14 @@ GemmPlan choose_plan(int64_t M, int64_t N, int64_t K, int cus) {
     const TileShape& s1 = kShapes[kPairs[pr][0]];
     const TileShape& s2 = kShapes[kPairs[pr][1]];
     const double d1 = tile_time(kPairs[pr][0], steps), d2 = tile_time(kPairs[pr][1], steps);
+    const int64_t rows1 = cdiv(M, s1.bm), rows2 = cdiv(M, s2.bm);
     for (int64_t k = cdiv(N, s1.bn); k >= 0; --k) {
       // no launch with a big tile ends before that tile: on to the small ones
       // alone (a few rows into 9216 columns: 4.4 us of host time a call -> 0.2)
-      if (k > 0 && d1 >= best_t * ahead) {
-        k = 1;
-        continue;
-      }
+      if (d1 >= best_t * ahead) k = 0;
       const int64_t n1 = std::min(k * s1.bn, N);
-      const int64_t t1 = cdiv(M, s1.bm) * cdiv(n1, s1.bn);
-      const int64_t t2 = cdiv(M, s2.bm) * cdiv(N - n1, s2.bn);
+      const int64_t t1 = rows1 * k;
+      const int64_t t2 = rows2 * ((uint32_t)(N - n1 + s2.bn - 1) / (uint32_t)s2.bn);
       // no order of the tiles ends before their total time shared by the CUs
       const double work = (double)cdiv(t1, 8) * d1 + (double)cdiv(t2, 8) * d2;
       if (launch_time(work / (double)P, work, P, steps) >= best_t * ahead) continue;
