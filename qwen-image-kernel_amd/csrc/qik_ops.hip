@@ -621,11 +621,17 @@ int launch_rope(int64_t D, bool fp16, RmsRopeParams& a, int64_t ga, RmsRopeParam
        {(const void*)rms_rope_pair_kernel<128, false>, (const void*)rms_rope_pair_kernel<128, true>}},
       {{(const void*)rms_rope_kernel<256, false>, (const void*)rms_rope_kernel<256, true>},
        {(const void*)rms_rope_pair_kernel<256, false>, (const void*)rms_rope_pair_kernel<256, true>}}};
+  // A single call of 128-wide heads runs the pair's kernel (all workgroups are
+  // a's) from seven workgroups per two CUs on: its instructions happen to be 1 to
+  // 2% faster there (2500 x 24 7.55 us against 7.65, 4352 x 24 11.3 / 11.45, 8000 x
+  // 24 19.1 / 19.3) and slower below (2000 x 24 6.36 / 6.32) and at the other head
+  // sizes (24 heads x 32 to x 256, 1000 to 8000 rows: 0 to 7%).
+  const bool pair = b != nullptr || (D == 128 && ga * 2 >= 7 * (int64_t)std::max(device_cus(), 1));
   int na = (int)ga;
   void* one[] = {&a};
-  void* both[] = {&a, b, &na};
-  const hipError_t e = hipLaunchKernel(fns[head_dim_index(D)][b != nullptr][fp16 ? 1 : 0], dim3((unsigned)(ga + gb)),
-                                       dim3(NTHREADS), b != nullptr ? both : one, 0, static_cast<hipStream_t>(stream));
+  void* both[] = {&a, b != nullptr ? b : &a, &na};
+  const hipError_t e = hipLaunchKernel(fns[head_dim_index(D)][pair ? 1 : 0][fp16 ? 1 : 0], dim3((unsigned)(ga + gb)),
+                                       dim3(NTHREADS), pair ? both : one, 0, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? QIK_OK : QIK_ERR_LAUNCH;
 }
 

@@ -74,6 +74,22 @@ def test_rms_rope_bit_exact_vs_oracle(B, S, H, D, dtype):
     assert (out.float() - ref.float()).abs().max().item() < 4e-2
 
 
+@pytest.mark.parametrize("S", [2380, 2400])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_rms_rope_large_call_equals_its_parts(S, dtype):
+    """Both sides of the line (on 256 CUs) from which a single call of 128-wide heads runs the
+    pair's kernel: every row as calls of a few hundred positions give it."""
+    _flush(f"case rms_rope large {S} {dtype}")
+    g = torch.Generator(device=DEV).manual_seed(S)
+    x = torch.randn(1, S, 72, 128, generator=g, device=DEV).to(dtype)[:, :, 24:48]
+    w = torch.randn(128, generator=g, device=DEV) * 0.3
+    freqs = orr.rope_freqs(S, 128).to(DEV)
+    got = qik.fused_rms_norm_rope(x, w, freqs, 1e-6)
+    for s0 in range(0, S, 700):
+        part = qik.fused_rms_norm_rope(x[:, s0:s0 + 700], w, freqs[s0:s0 + 700], 1e-6)
+        np.testing.assert_array_equal(_bits(got[:, s0:s0 + 700]), _bits(part))
+
+
 def test_rms_rope_reads_fused_qkv_views_in_place():
     """q/k as strided slices of a fused QKV output (processors.py:65-70)."""
     _flush("case rms_rope strided")
